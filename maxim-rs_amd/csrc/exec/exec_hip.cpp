@@ -21,6 +21,7 @@
 #include <mutex>
 #include <set>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../hip/kargs.h"
@@ -745,18 +746,22 @@ private:
         if (a.K % 16 || a.N % 4 || a.K == 0 || wout <= 0 || slen <= 0) return false;
         if (!aligned(a.A, 16) || !aligned(a.B, 16) || !aligned(a.C, 16)) return false;
         if (layout == 1 && !aligned(a.bias, 16)) return false;
+        const auto parts = w3.find({a.A, wout, (int64_t)a.K});
+        if (parts == w3.end() || a.sA) return false;
+        a.A3 = wdev + parts->second;
         if (a.sA % 4 || a.sB % 4 || a.sC % 4 || a.batch > 65535) return false;
         static const char *names[2][3] = {{"mx_pw_ch1", "mx_pw_ch2", "mx_pw_ch4"},
                                           {"mx_pw_rw1", "mx_pw_rw2", "mx_pw_rw4"}};
-        // Tile width and reduction split, from measurements on MI355X: 32
-        // weight outputs per wave in both layouts (64 for the row-major
-        // form's long reductions reused each operand load twice as often
-        // but held 186 VGPRs, two waves per SIMD: the GateMm mode-1 launches
-        // run 2-7% faster at 32 at 224x320 and the same at 448x640; the
-        // channel-major form is 3-12% faster at 32 for 1x1 convs of 256-512
-        // inputs and GateMm over 256 tokens); the block's four waves split
-        // reductions of 128 and more, and shorter ones when one wave per
-        // tile would leave SIMDs idle.
+        // Tile width, sharing and reduction split, from measurements on
+        // MI355X: 32 weight outputs per wave in both layouts; four (two)
+        // waves share X where the weight tiles come in fours (twos), so X is
+        // split once for 128 (64) outputs. With at least one tile per SIMD
+        // that is the faster form (c -> c 1x1 convs of 128 channels at 112x160,
+        // 1120 tiles: 9.4 us against 10.7 with the split reduction; GateMm over
+        // 64 tokens, 128 channels at 112x160: 6.8 against 10.5); below it the
+        // block's four waves split the reduction (56x80, 280 tiles: 4.6 us
+        // against 6.0; a 64x64 pass 1.83 ms against 2.35). A reduction of 128
+        // and more that no waves can share X of is split too.
         const int ti = wout <= 16 ? 0 : 1, tmw = 1 << ti;
         const int64_t nib = (wout + 16 * tmw - 1) / (16 * tmw);
         const int64_t tiles = nib * ((slen + 63) / 64);
@@ -765,8 +770,9 @@ private:
         // normalises bands across several waves of a block, which needs them
         // to hold whole tiles)
         const int64_t nbat = fold ? 1 : a.batch;
-        const bool k4 = !whole && a.K % 64 == 0 && (a.K >= 128 || tiles * nbat < 2LL * 4 * cus);
-        l = mk(std::string(names[layout][ti]).insert(8, fold ? "b" : "") + (k4 ? "_k4" : ""));
+        const char *sh = shared_x(nib, a.K);
+        const bool k4 = !whole && a.K % 64 == 0 && ((a.K >= 128 && !*sh) || tiles * nbat < 4LL * cus);
+        l = mk(std::string(names[layout][ti]).insert(8, fold ? "b" : "") + (k4 ? "_k4" : sh));
         const int64_t grid = k4 ? tiles : (tiles + 3) / 4;
         if (grid > 0x7fffffffLL) return false;
         l.g[0] = (unsigned)grid;
@@ -775,6 +781,14 @@ private:
         set_args(l, a);
         return true;
     }
+    // The form in which waves holding tiles of the same streamed elements share
+    // X (pointwise.h, SH): nib weight tiles per column block, four (or two)
+    // waves to a group, whole stages of 16 k's a wave.
+    static const char *shared_x(int64_t nib, int64_t k) {
+        return nib % 4 == 0 && k % 64 == 0 ? "_s4" : nib % 2 == 0 && k % 32 == 0 ? "_s2" : "";
+    }
+    // (weight matrix, rows, k's) -> its bf16 parts (GemmArgs A3), a byte offset in wdev
+    std::map<std::tuple<const float *, int64_t, int64_t>, uint64_t> w3;
     std::vector<std::vector<Launch>> alt;
     std::vector<char> whole_k;  // per op: keep a streaming GEMM's reduction in one wave
     bool no_pw = getenv("MAXIM_NO_PW") != nullptr;
@@ -1057,6 +1071,29 @@ void Gpu::init(const mx_plan_desc *p) {
         }
     }
     blob.resize((blob.size() + 63) & ~(size_t)63);
+    // The weights of the streaming GEMMs again, as the bf16 parts their kernels
+    // multiply: six bytes an element, split on the device from the blob.
+    struct Parts {
+        int64_t off, rows, k;
+        uint64_t at;
+    };
+    std::vector<Parts> parts;
+    wbytes = blob.size() * 4;
+    {
+        std::set<std::array<int64_t, 3>> seen;
+        auto add = [&](int64_t off, int64_t rows, int64_t k) {
+            if (off < 0 || rows <= 0 || k <= 0 || k % 16 || !seen.insert({off, rows, k}).second) return;
+            if (rows > 0x7fffffff || k > 0x7fffffff) return;
+            parts.push_back(Parts{off, rows, k, wbytes});
+            wbytes += (uint64_t)((rows + 15) / 16 * ((k + 31) / 32)) * 3072;
+        };
+        for (uint64_t i = 0; i < p->n_ops; ++i) {
+            const mx_op &o = p->ops[i];
+            if (o.kind == MX_OP_CONV1X1 && o.h * o.wd > 1) add(woff[o.w], o.c_out, o.c_in);
+            if (o.kind == MX_OP_CONVT2X2) add(extra[i][1], 4 * o.c_out, o.c_in);
+            if (o.kind == MX_OP_GATE_MM) add(woff[o.w], o.p[o.mode == 0 ? 0 : 1], o.p[o.mode == 0 ? 0 : 1]);
+        }
+    }
 
     // The fused program and the device layout it implies.
     n_ops = p->n_ops;
@@ -1087,7 +1124,6 @@ void Gpu::init(const mx_plan_desc *p) {
     }
 
     // Size the pass before allocating it, and refuse with the numbers.
-    wbytes = blob.size() * 4;
     // Scratch: channel-mean partial sums, then the statistics of a folded
     // LayerNorm ([2][hw], one step at a time).
     ln_off = (mean_scratch + 63) & ~(uint64_t)63;
@@ -1132,7 +1168,17 @@ void Gpu::init(const mx_plan_desc *p) {
     wdev = static_cast<unsigned char *>(ptr);
     check(H.hipMalloc(&ptr, scratch_len * 4), "hipMalloc(scratch)");
     scratch = static_cast<float *>(ptr);
-    if (wbytes) check(H.hipMemcpy(wdev, blob.data(), wbytes, kMemcpyH2D), "hipMemcpy(weights)");
+    if (!blob.empty()) check(H.hipMemcpy(wdev, blob.data(), blob.size() * 4, kMemcpyH2D), "hipMemcpy(weights)");
+    for (const Parts &q : parts) {
+        const float *w = reinterpret_cast<const float *>(wdev) + q.off;
+        Launch l = mk("mx_split_w");
+        set_args(l, SplitArgs{w, wdev + q.at, (int32_t)q.rows, (int32_t)q.k});
+        l.g[0] = cdiv(q.rows, 16);
+        launch(l);
+        w3[{w, q.rows, q.k}] = q.at;
+    }
+    kernels = 0;
+    sync();
     if (std::getenv("MAXIM_LOG_ALLOC"))
         fprintf(stderr, "maxim: arena [%p, %p) weights [%p, %p) scratch [%p, %p) static scratch [%p, %p)\n",
                 (void *)arena, (void *)(arena + arena_len), (void *)wdev, (void *)(wdev + wbytes), (void *)scratch,
@@ -2501,8 +2547,8 @@ void Gpu::build_program(const mx_plan_desc *p) {
             GemmArgs a;
             memcpy(&a, l.a0, sizeof a);
             if (a.M <= 32 && a.batch == 1) {
-                const int64_t tiles = (int64_t)((a.M + 15) / 16) * ((a.N + 63) / 64);
-                l.name = intern(std::string("mx_pw_ch1") + (l.name + 9));
+                const int64_t nib = (a.M + 15) / 16, tiles = nib * ((a.N + 63) / 64);
+                l.name = intern(std::string("mx_pw_ch1") + shared_x(nib, a.K) + (l.name + 9));
                 l.f = fn(l.name);
                 l.g[0] = (unsigned)((tiles + 3) / 4);
             }
@@ -2609,9 +2655,9 @@ void Gpu::build_program(const mx_plan_desc *p) {
         GemmArgs a;
         memcpy(&a, l.a0, sizeof a);
         if (a.batch != 1 || (mode == 0 && a.ymap.on) || (need_ymap && !a.ymap.on)) return false;
-        // the name is mx_pw_ch<T>[_k4][_ln][_f]: nothing else may be folded in
+        // the name is mx_pw_ch<T>[_k4|_s2|_s4][_ln][_f]: nothing else may be folded in
         std::string rest = nm.substr(9);
-        for (const char *t : {"_k4", "_ln", "_f"})
+        for (const char *t : {"_k4", "_s2", "_s4", "_ln", "_f"})
             if (!rest.compare(0, strlen(t), t)) rest = rest.substr(strlen(t));
         if (!rest.empty() || r0 < 0 || r0 % c || r0 + nband * c > a.M) return false;
         // y may overlap nothing the kernel reads or writes
@@ -2644,8 +2690,9 @@ void Gpu::build_program(const mx_plan_desc *p) {
             G = 1;
         }
         if (!G) return false;
-        const int64_t tiles = ((a.M + 16 * tmw - 1) / (16 * tmw)) * ((a.N + 63) / 64);
-        l.name = intern("mx_pw_ch" + std::to_string(tmw) + (k4 ? "_k4" : "") + (lnn ? "_ln" : "") + "_f_lo");
+        const int64_t nib = (a.M + 16 * tmw - 1) / (16 * tmw), tiles = nib * ((a.N + 63) / 64);
+        l.name = intern("mx_pw_ch" + std::to_string(tmw) + (k4 ? "_k4" : tmw > 2 || (tmw == 1 && lnn) ? "" : shared_x(nib, a.K)) +
+                        (lnn ? "_ln" : "") + "_f_lo");
         l.f = fn(l.name);
         l.g[0] = (unsigned)(k4 ? tiles : (tiles + 3) / 4);
         l.g[1] = 1;

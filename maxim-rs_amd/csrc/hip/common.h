@@ -14,6 +14,55 @@ __device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// fp32 products on the bf16 matrix cores. A float splits exactly into three
+// bf16 parts, x = h + m + l (8 + 8 + 8 significand bits, each part the rounded
+// remainder of the last), and of the nine products of two split floats the six
+// of order 2^0, 2^-8 and 2^-16 are kept; what is dropped is below 2^-24 of the
+// product. Each v_mfma_f32_16x16x32_bf16 adds 32 exact products in fp32 with
+// one rounding, so a sum of K products is rounded 6 K / 32 times where the
+// fp32 MFMA chain rounds K times: against 64-bit sums of N(0, 1) products the
+// relative error is 3.7e-8 / 9.2e-8 / 1.5e-7 / 2.3e-7 at K = 32 / 64 / 128 /
+// 256, the fp32 MFMA's 1.0e-7 / 1.4e-7 / 2.0e-7 / 2.9e-7. Six bf16 MFMAs take
+// 96 cycles of a SIMD for the 32 k's that eight fp32 ones take 256 for, and
+// leave most of the vector ALU's issue slots free (the fp32 MFMA does not).
+// Parts below 2^-126 are flushed, so operands under 2^-110 lose their last
+// parts; an infinite, NaN or over-2^127.99 operand gives NaN in every product,
+// and a wave that finds a non-finite sum computes its tile again in fp32.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// Two floats as packed bf16, rounded to nearest even.
+__device__ __forceinline__ uint32_t bf2(float a, float b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+// The three parts of two floats, packed in pairs: 3.5 vector operations per
+// element, the remainders by the packed dot product with (-1, 0) and (0, -1)
+// (exact: a remainder is a float). The constants come through registers,
+// since the instruction's inline -1 is not a packed pair.
+__device__ __forceinline__ void split2(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l) {
+    uint32_t c0, c1;
+    asm("s_mov_b32 %0, 0xbf80" : "=s"(c0));
+    asm("s_mov_b32 %0, 0xbf800000" : "=s"(c1));
+    const bf16x2 n0 = __builtin_bit_cast(bf16x2, c0), n1 = __builtin_bit_cast(bf16x2, c1);
+    h = bf2(a, b);
+    const bf16x2 hv = __builtin_bit_cast(bf16x2, h);
+    const float r0 = __builtin_amdgcn_fdot2_f32_bf16(hv, n0, a, false);
+    const float r1 = __builtin_amdgcn_fdot2_f32_bf16(hv, n1, b, false);
+    m = bf2(r0, r1);
+    const bf16x2 mv = __builtin_bit_cast(bf16x2, m);
+    l = bf2(__builtin_amdgcn_fdot2_f32_bf16(mv, n0, r0, false), __builtin_amdgcn_fdot2_f32_bf16(mv, n1, r1, false));
+}
+// One 16x16x32 bf16 MFMA: lane l supplies eight k's of A's row l % 16 and of
+// B's column l % 16 (which eight is the caller's, the same for both), the
+// accumulator laid out as mfma16's.
+__device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                   0, 0);
+}
+
 // Work-group placement. The dispatcher deals consecutive work-group ids to
 // the 8 XCDs in turn, and each XCD has its own L2, so neighbouring tiles
 // (which share halo rows, cache lines and operands) land in different L2s.

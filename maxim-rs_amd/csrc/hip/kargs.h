@@ -227,6 +227,17 @@ struct GemmArgs {
     // The grid is then one-dimensional.
     int32_t fold, fsh;
     uint32_t fmul, pad2;
+    const void *A3;       // the streaming kernels' weights, A split into bf16 parts (SplitArgs)
+};
+
+// A weight matrix [M][K] as the bf16 matrix cores' operands: each element's
+// three bf16 parts, [ceil(M / 16)][ceil(K / 32)][part][lane][8], lane l
+// holding row 16 t + l % 16 at k = 32 c + 4 (l / 16) + 0..3 and 16 more
+// (zeros past M and K).
+struct SplitArgs {
+    const float *w;
+    void *out;
+    int32_t M, K;
 };
 
 // Two independent streaming-GEMM launches of one kernel in one grid: blocks

@@ -1,10 +1,10 @@
-// Streaming fp32 MFMA kernels for the Dense-shaped ops whose reduction is
+// Streaming matrix-core kernels for the Dense-shaped ops whose reduction is
 // short next to their streamed axis: every 1x1 conv (K = c_in <= 512 over
-// up to 286720 pixels) and both GateMm modes. Operands go straight from
-// memory into the matrix cores with 128-bit loads (no LDS staging): each wave
-// owns a 64 x (16 * TMW) output tile, or a quarter of its reduction, so a CU
-// keeps many independent waves in flight and the epilogue of one overlaps
-// the loads of another.
+// up to 286720 pixels) and both GateMm modes. Products of floats are formed
+// from three-part bf16 operands (common.h): the weights split once, at upload
+// (GemmArgs A3), the streamed operand X in registers on its way to the matrix
+// cores. Each wave owns a 64 x (16 * TMW) output tile, or a quarter of its
+// reduction.
 //
 // Two layouts share one body (D = the 16x16 MFMA tile, lane l = 16g + i):
 //
@@ -18,9 +18,19 @@
 //       A operand = W, B operand = X^T, so a lane holds four consecutive
 //       outputs of one row: D[4g + r][i] = Y[n0 + 16j + i][a0 + 4g + r].
 //
-// The reduction runs in supersteps of 16: within one, lane group g supplies
-// k = 16 S + 4 g + t at MFMA step t, which covers the 16 k's exactly once and
-// lets each lane fetch its four k's of a row with one 128-bit load.
+// X is loaded in supersteps of 16 k's: lane group g supplies k = 16 S + 4 g + t,
+// t = 0..3, so each lane fetches its four k's of a row with one 128-bit load.
+// Two supersteps make the 32 k's of an MFMA, whatever their order, as the
+// weights are laid out in the same one. The six products of every 32 k's are
+// added smallest first, and the 32s in ascending order, in every form of the
+// kernel, so forms that differ in tile width or in how X reaches the matrix
+// cores agree to the bit.
+//
+// Measured on MI355X against the same kernels on fp32 MFMAs (which are bound by
+// the SIMDs' issue: MFMA and VALU add up there): GateMm over 256 tokens, 32
+// channels at 448x640, 60.2 -> 34.4 us (mode 0) and 66.1 -> 34.1 us (mode 1),
+// 137 TFLOP/s; LayerNorm + Dense 128 -> 256 + GELU at 112x160 24.2 -> 14.7 us,
+// 32 -> 64 at 448x640 28.0 -> 23.0 us; a 640x448 S-3 pass 22.8 -> 19.5 ms.
 #pragma once
 
 #include "common.h"
@@ -44,12 +54,18 @@ __device__ __forceinline__ float comp(const float4 &v, int t) {
 // tile's reduction into quarters and add the partial sums in LDS in a fixed
 // order (wave 0 + 1 + 2 + 3), for the shapes with too few tiles to fill the
 // chip.
+// SH (KS = 1): SH consecutive waves of a block hold weight tiles of the same
+// 64 streamed elements (the tile count per column block is a multiple of SH)
+// and share X: per stage of 16 SH k's each wave loads one superstep, normalises
+// and splits it once, and leaves the parts in LDS for all of them (24 KB a
+// block), so an element of X is loaded, normalised and split once for 16 TMW SH
+// outputs instead of 16 TMW. SH = 1: each wave feeds its own registers.
 //
 // Operand loads are clamped into range instead of guarded: an X column or
 // weight row past the edge only feeds output rows/columns of the MFMA tile
 // that are never stored, so no branch or select sits between the loads and
-// the matrix cores. The reduction ping-pongs between two register buffers,
-// so the loads of superstep s + 1 are in flight while superstep s multiplies.
+// the matrix cores. The next stage's (or 32 k's) loads are in flight while one
+// multiplies.
 // The image index of blocked index e (0 <= e < plane) under map q (32-bit:
 // the host enables a map only below 2^31 elements).
 // n / d for n < 2^31, with the host's multiplier m and shift s for d.
@@ -79,11 +95,11 @@ enum { EP_U = 1, EP_R1 = 2, EP_R2 = 4, EP_GELU = 8, EP_LRELU = 16, EP_YMAP = 32,
 // waves in turn), so its normalised X differs from theirs by rounding.
 // (ux, nx): this block's index and the block count along x, by: the batch;
 // a kernel pairing two launches in one grid passes each part its own.
-// XR: the split reduction's LDS buffer comes from the caller (xred, 4 x 16
-// TMW x 64 floats), so two different instances in one kernel share one.
+// XR: the LDS pool comes from the caller (xpool, as many floats as `POOL`
+// below), so two different instances in one kernel share one.
 template <int LAYOUT, int TMW, int KS, bool FUSED, int LN, bool XM = false, bool XMUL = false, bool CT = false,
-          bool LNO = false, int EP = -1, bool FOLD = false, bool XR = false>
-__device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xred = nullptr) {
+          bool LNO = false, int EP = -1, bool FOLD = false, bool XR = false, int SH = 1>
+__device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = nullptr) {
     const bool has_u = EP < 0 ? a.e.u != nullptr : (EP & EP_U) != 0;
     const bool has_r1 = EP < 0 ? a.e.r1 != nullptr : (EP & EP_R1) != 0;
     const bool has_r2 = EP < 0 ? a.e.r2 != nullptr : (EP & EP_R2) != 0;
@@ -107,7 +123,7 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xred = nu
     const int nib = (wout + TW - 1) / TW;
     const int ntiles = nib * ((slen + 63) / 64);  // < 2^31, checked by the host
     const int b = fold ? 0 : by;
-    const float *W = a.A + (int64_t)b * a.sA;
+    const float *W = a.A;
     const float *X = a.B + (int64_t)b * a.sB;
     float *Y = a.C + (int64_t)b * a.sC;
     // X's advance per superstep (16 k's): 16 rows (CH) or 16 columns (RW);
@@ -122,18 +138,18 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xred = nu
     const int nb = nx;
     if ((nb & 7) == 0) unit = (unit & 7) * (nb >> 3) + (unit >> 3);
     const int tile = KS == 1 ? unit * 4 + wave : unit;
-    if (tile >= ntiles) return;  // KS = 4: the whole block
+    static_assert(SH == 1 || KS == 1, "X is shared by waves with whole reductions");
+    // KS = 4: the whole block; SH > 1: waves past the last tile stay for the
+    // block's barriers (their columns lie past the edge, nothing is stored)
+    if (SH == 1 && tile >= ntiles) return;
     const int nS = K / 16;
-    const int S0 = KS == 1 ? 0 : wave * (nS / 4);
-    const int nSw = KS == 1 ? nS : nS / 4;  // supersteps of this wave
+    // this wave's first superstep: of its share of the reduction (KS = 4), of
+    // its share of each stage (SH > 1)
+    const int S0 = SH > 1 ? wave % SH : KS == 1 ? 0 : wave * (nS / 4);
+    const int nSw = KS == 1 ? nS : nS / 4;  // supersteps of this wave's reduction
 
     const int w0 = (tile % nib) * TW;
     const int s0 = (tile / nib) * 64;
-    // This lane's operand streams at the wave's first superstep.
-    const float *wp[TMW];
-#pragma unroll
-    for (int mt = 0; mt < TMW; ++mt)
-        wp[mt] = W + (int64_t)min(w0 + mt * 16 + i, wout - 1) * K + 4 * g + S0 * 16;
     // Input maps: X as the blocked view of an image-ordered tensor (an
     // elided forward permutation). With a folded LayerNorm (CH, xmap.on): X
     // is [channels][pixels] and only the pixel axis is blocked. XM (GateMm):
@@ -199,15 +215,14 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xred = nu
     const float *xq[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) xq[q] = XMUL ? a.B2 + (int64_t)b * a.sB + (xp[q] - X) : nullptr;
-    auto load = [&](int s, float4 *xv, float4 *wv, float4 *lv, float4 *mv) {
+    // superstep S0 + s of X, with what its normalisation or product needs
+    auto load = [&](int s, float4 *xv, float4 *lv, float4 *mv) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) xv[q] = ld4(xp[q] + s * xstep);
         if (XMUL) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) mv[q] = ld4(xq[q] + s * xstep);
         }
-#pragma unroll
-        for (int mt = 0; mt < TMW; ++mt) wv[mt] = ld4(wp[mt] + s * 16);
         if (LN) {
             lv[0] = ld4(lsc + s * 16);
             lv[1] = ld4(lbi + s * 16);
@@ -223,11 +238,10 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xred = nu
             xv[q].w = (xv[q].w - lmean.w) * lrstd.w * w + c;
         }
     };
-    // first: the wave's first superstep, whose multiplies start from zero
-    // (an inline-constant accumulator instead of 16 TMW register moves)
-    auto mma = [&](float4 *xv, const float4 *wv, const float4 *lv, const float4 *mv, bool first) {
+    // the loaded values to X's: normalised, or multiplied (mx_mul's a * b)
+    auto ready = [&](float4 *xv, const float4 *lv, const float4 *mv) {
         if (LN) norm(xv, lv);
-        if (XMUL) {  // mx_mul's a * b
+        if (XMUL) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 xv[q].x = xv[q].x * mv[q].x;
@@ -236,19 +250,57 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xred = nu
                 xv[q].w = xv[q].w * mv[q].w;
             }
         }
+    };
+    // the superstep's four k's of streamed element j of this lane, split
+    struct Half {
+        uint32_t h[2], m[2], l[2];
+    };
+    auto split = [&](const float4 *xv, int j) {
+        Half o;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            if (LAYOUT == CH)
+                split2(comp(xv[2 * t], j), comp(xv[2 * t + 1], j), o.h[t], o.m[t], o.l[t]);
+            else
+                split2(comp(xv[j], 2 * t), comp(xv[j], 2 * t + 1), o.h[t], o.m[t], o.l[t]);
+        }
+        return o;
+    };
+    // the weight parts of 32 k's (chunk c) for this wave's outputs
+    const int nC = (K + 31) / 32;
+    const u32x4 *w3[TMW];
+#pragma unroll
+    for (int mt = 0; mt < TMW; ++mt)
+        w3[mt] = (const u32x4 *)a.A3 + (int64_t)min(w0 / 16 + mt, (wout + 15) / 16 - 1) * nC * 192 + lane;
+    struct WParts {
+        u32x4 p[TMW][3];
+    };
+    auto wload = [&](int c) {
+        WParts w;
+#pragma unroll
+        for (int mt = 0; mt < TMW; ++mt)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) w.p[mt][q] = w3[mt][(c * 3 + q) * 64];
+        return w;
+    };
+    // the six products of streamed tile j's 32 k's with the weights, smallest
+    // first; first: the wave's first 32, which start from zero (an
+    // inline-constant accumulator instead of register moves)
+    auto mul = [&](int j, u32x4 xh, u32x4 xm, u32x4 xl, const WParts &w, bool first) {
         const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        auto one = [&](u32x4 x, int q, bool z) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int mt = 0; mt < TMW; ++mt) {
-                    const f32x4 c = first && t == 0 ? zero : acc[j][mt];
-                    if (LAYOUT == CH)
-                        acc[j][mt] = mfma16(comp(xv[t], j), comp(wv[mt], t), c);
-                    else
-                        acc[j][mt] = mfma16(comp(wv[mt], t), comp(xv[j], t), c);
-                }
+            for (int mt = 0; mt < TMW; ++mt) {
+                const f32x4 c = z ? zero : acc[j][mt];
+                acc[j][mt] = LAYOUT == CH ? mfma32(x, w.p[mt][q], c) : mfma32(w.p[mt][q], x, c);
+            }
+        };
+        one(xh, 2, first);
+        one(xl, 0, false);
+        one(xm, 1, false);
+        one(xh, 1, false);
+        one(xm, 0, false);
+        one(xh, 0, false);
     };
     // The bias of this lane's outputs, fetched before the reduction.
     float4 bias[TMW];
@@ -262,11 +314,17 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xred = nu
         else bias[mt] = ld4(a.bias + min(w0 + mt * 16 + 4 * g, wout - 4));
     }
 
-    float4 xa[4], wa[TMW], la[2], ma[4], xb[4], wb[TMW], lb[2], mb[4];
-    // Loads are unconditional (past the wave's last superstep they re-read
-    // it), so the wait before each multiply counts only the loads it needs.
-    load(0, xa, wa, la, ma);
-    load(min(1, nSw - 1), xb, wb, lb, mb);
+    // SH = 1: the two supersteps of the wave's first 32 k's (loads are
+    // unconditional, a superstep outside the wave's share re-reads an end of
+    // it and is zeroed); SH > 1: its superstep of the first stage.
+    float4 xa[4], la[2], ma[4], xb[4], lb[2], mb[4];
+    const int par = SH == 1 ? S0 & 1 : 0;  // the share starts at the second superstep of a chunk
+    if (SH == 1) {
+        load(0, xa, la, ma);
+        load(min(1 - par, nSw - 1), xb, lb, mb);
+    } else {
+        load(0, xa, la, ma);
+    }
     if constexpr (LN == 2) {
         static_assert(KS == 4 && LAYOUT == CH, "in-kernel statistics: the split-reduction channel-major form");
         // This lane's rows k = 16 S + 4 g + q of its two supersteps (xa, xb)
@@ -387,18 +445,136 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xred = nu
         operands(0, 0);
         if (NK > 1) operands(1, 1);
     }
-    mma(xa, wa, la, ma, true);
-    int s = 1;
-    for (; s + 2 <= nSw; s += 2) {
-        load(s + 1, xa, wa, la, ma);
-        mma(xb, wb, lb, mb, false);
-        load(min(s + 2, nSw - 1), xb, wb, lb, mb);
-        mma(xa, wa, la, ma, false);
+    // LNO: the wave whose tile is the output LayerNorm's channels keeps its
+    // final values for it (and stores them raw only when asked to): with
+    // KS = 1 in its own rows of LDS at once, with KS = 4 (where LDS still
+    // holds the partial sums) in registers until every wave has read them.
+    constexpr int PC = KS == 1 ? 64 : 16;  // pixel columns of a wave's tile
+    constexpr int LDT = PC + 4;            // padded LDS row
+    constexpr int PER = TW * LDT + 2 * PC;  // LDS floats per wave
+    // one LDS pool: X's parts, then the split reduction's partial sums or the
+    // output LayerNorm's tiles
+    constexpr int STAGE = SH > 1 ? 4 * 64 * 24 : 0, RED = KS == 4 ? 4 * NACC * 64 : 0;
+    constexpr int TILES = LNO && KS == 1 ? 4 * PER : 0;
+    constexpr int POOL = STAGE > RED ? (STAGE > TILES ? STAGE : TILES) : (RED > TILES ? RED : TILES);
+    __shared__ __align__(16) float pool_own[XR || POOL == 0 ? 4 : POOL];
+    float *const pool = XR ? xpool : pool_own;
+    if constexpr (SH == 1) {
+        // chunk cc of the wave's share: supersteps 2 cc - par and the next
+        const int nc = (nSw + par + 1) / 2, c0 = S0 >> 1;
+        const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        auto step = [&](int cc, bool first) {
+            const WParts w = wload(c0 + cc);
+            ready(xa, la, ma);
+            ready(xb, lb, mb);
+            if (first && par) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) xa[q] = zero4;
+            }
+            if (2 * cc + 1 - par >= nSw) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) xb[q] = zero4;
+            }
+            u32x4 xs[4][3];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const Half p = split(xa, j), q = split(xb, j);
+                xs[j][0] = u32x4{p.h[0], p.h[1], q.h[0], q.h[1]};
+                xs[j][1] = u32x4{p.m[0], p.m[1], q.m[0], q.m[1]};
+                xs[j][2] = u32x4{p.l[0], p.l[1], q.l[0], q.l[1]};
+            }
+            if (cc + 1 < nc) {
+                load(2 * cc + 2 - par, xa, la, ma);
+                load(min(2 * cc + 3 - par, nSw - 1), xb, lb, mb);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) mul(j, xs[j][0], xs[j][1], xs[j][2], w, first);
+        };
+        step(0, true);
+#pragma unroll 1
+        for (int cc = 1; cc < nc; ++cc) step(cc, false);
+    } else {
+        // The parts of a stage in LDS: [chunk][part][lane group g][64 streamed
+        // elements][8 k's], 16 bytes a lane, tile j's sixteen side by side;
+        // superstep S fills the half S % 2 of chunk S / 2. Each group of SH
+        // waves has its own.
+        constexpr int SC = SH / 2;  // chunks per stage
+        unsigned char *const sx = (unsigned char *)pool + (wave / SH) * (SH * 6144);
+        unsigned char *const wr = sx + ((S0 >> 1) * 12 + g) * 1024 + i * 16 + (S0 & 1) * 8;
+        const unsigned char *const rd = sx + g * 1024 + i * 16;
+        const int nst = nS / SH;
+        auto stage = [&](int st, bool first) {
+            WParts w = wload(st * SC);
+            ready(xa, la, ma);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const Half p = split(xa, j);
+                *(uint2 *)(wr + j * 256) = make_uint2(p.h[0], p.h[1]);
+                *(uint2 *)(wr + 4096 + j * 256) = make_uint2(p.m[0], p.m[1]);
+                *(uint2 *)(wr + 8192 + j * 256) = make_uint2(p.l[0], p.l[1]);
+            }
+            __syncthreads();
+            WParts wn = w;
+            if (SC > 1) wn = wload(st * SC + 1);
+            if (st + 1 < nst) load((st + 1) * SH, xa, la, ma);
+#pragma unroll
+            for (int cc = 0; cc < SC; ++cc) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const unsigned char *r = rd + cc * 12288 + j * 256;
+                    mul(j, *(const u32x4 *)r, *(const u32x4 *)(r + 4096), *(const u32x4 *)(r + 8192), cc ? wn : w,
+                        first && cc == 0);
+                }
+            }
+        };
+        stage(0, true);
+#pragma unroll 1
+        for (int st = 1; st < nst; ++st) {
+            __syncthreads();  // every wave has read the last stage's parts
+            stage(st, false);
+        }
+        if (LNO) __syncthreads();
     }
-    if (s < nSw) mma(xb, wb, lb, mb, false);
+    // An operand the split cannot hold (infinite, NaN, the largest floats)
+    // leaves NaN in its outputs, and sums may overflow: a wave with any
+    // non-finite sum forms its sums in fp32 instead, superstep by superstep.
+    float fin = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int mt = 0; mt < TMW; ++mt) {
+            fin = __builtin_fmaf(acc[j][mt][0], acc[j][mt][1], fin);
+            fin = __builtin_fmaf(acc[j][mt][2], acc[j][mt][3], fin);
+        }
+    if (__builtin_amdgcn_ballot_w64(!__builtin_isfinite(fin))) {
+        const int first = SH > 1 ? -S0 : 0;
+        const float *wp[TMW];
+#pragma unroll
+        for (int mt = 0; mt < TMW; ++mt)
+            wp[mt] = W + (int64_t)min(w0 + mt * 16 + i, wout - 1) * K + 4 * g + (S0 + first) * 16;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int mt = 0; mt < TMW; ++mt) acc[j][mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (int s = 0; s < nSw; ++s) {
+            float4 wv[TMW];
+            load(first + s, xa, la, ma);
+#pragma unroll
+            for (int mt = 0; mt < TMW; ++mt) wv[mt] = ld4(wp[mt] + s * 16);
+            ready(xa, la, ma);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int mt = 0; mt < TMW; ++mt)
+                        acc[j][mt] = LAYOUT == CH ? mfma16(comp(xa[t], j), comp(wv[mt], t), acc[j][mt])
+                                                  : mfma16(comp(wv[mt], t), comp(xa[j], t), acc[j][mt]);
+        }
+    }
 
-    __shared__ float red_own[KS == 1 || XR ? 1 : 4 * NACC * 64];
-    float *const red = XR ? xred : red_own;
+    float *const red = pool;
     if (KS == 4) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -409,14 +585,7 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xred = nu
                     red[((wave * NACC) + (j * TMW + mt) * 4 + r) * 64 + lane] = acc[j][mt][r];
         __syncthreads();
     }
-    // LNO: the wave whose tile is the output LayerNorm's channels keeps its
-    // final values for it (and stores them raw only when asked to): with
-    // KS = 1 in its own rows of LDS at once, with KS = 4 (where LDS still
-    // holds the partial sums) in registers until every wave has read them.
-    constexpr int PC = KS == 1 ? 64 : 16;  // pixel columns of a wave's tile
-    constexpr int LDT = PC + 4;            // padded LDS row
-    constexpr int PER = TW * LDT + 2 * PC;  // LDS floats per wave
-    __shared__ float lt[LNO && KS == 1 ? 4 * PER : 1];
+    float *const lt = pool;
     const int lnspan = (KS == 1 ? a.lo.group : 1) * TW * a.lo.nband;  // rows with a LayerNorm
     const bool lnw = LNO && w0 >= a.lo.row0 && w0 < a.lo.row0 + lnspan;
     float4 vs[LNO && KS == 4 ? NK : 1];
@@ -668,53 +837,71 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xred = nu
 
 }  // namespace pw
 
-// mx_pw_{ch,rw}<TMW>[_k4][_ln|_xm|_mul][_f]: 256 threads; _k4 splits the
-// reduction over the block's four waves, _ln folds a channel LayerNorm into X
+// mx_pw_{ch,rw}<TMW>[_k4|_s2|_s4][_ln|_xm|_mul][_f]: 256 threads; _k4 splits the
+// reduction over the block's four waves, _s<SH> shares X between SH of them, _ln folds a channel LayerNorm into X
 // (CH only), _xm reads X through a token map (GateMm over an elided forward
 // permutation), _mul forms X as the product of two tensors (a folded Mul, CH
 // only), _f applies the fused epilogue. mx_pw_ch<TMW>[_k4]_t: the transposed
 // 2x2 stride-2 conv (rows ordered (ky, oc, kx), co and the input width in
 // GemmArgs co / wd, wd % 4 == 0).
-#define MXK_PW2(LNAME, LAYOUT, TMW, KS, LN, XM, XMUL, SUF)                                         \
+#define MXK_PW3(LNAME, LAYOUT, TMW, KS, LN, XM, XMUL, SH, SUF)                                     \
     extern "C" __global__ __launch_bounds__(256) void mx_pw_##LNAME##TMW##SUF(GemmArgs a) {        \
-        pw::body<pw::LAYOUT, TMW, KS, false, LN, XM, XMUL>(a, blockIdx.x, gridDim.x, blockIdx.y);                                     \
-    }                                                                                               \
+        pw::body<pw::LAYOUT, TMW, KS, false, LN, XM, XMUL, false, false, -1, false, false, SH>(    \
+            a, blockIdx.x, gridDim.x, blockIdx.y);                                                 \
+    }                                                                                              \
     extern "C" __global__ __launch_bounds__(256) void mx_pw_##LNAME##TMW##SUF##_f(GemmArgs a) {    \
-        pw::body<pw::LAYOUT, TMW, KS, true, LN, XM, XMUL>(a, blockIdx.x, gridDim.x, blockIdx.y);                                      \
+        pw::body<pw::LAYOUT, TMW, KS, true, LN, XM, XMUL, false, false, -1, false, false, SH>(     \
+            a, blockIdx.x, gridDim.x, blockIdx.y);                                                 \
     }
+#define MXK_PW2(LNAME, LAYOUT, TMW, KS, LN, XM, XMUL, SUF) MXK_PW3(LNAME, LAYOUT, TMW, KS, LN, XM, XMUL, 1, SUF)
 #define MXK_PW1(LNAME, LAYOUT, TMW, KS, LN, XM, SUF) MXK_PW2(LNAME, LAYOUT, TMW, KS, LN, XM, false, SUF)
+// _s<SH>: X shared by SH waves of a block
+#define MXK_PW_S(LNAME, LAYOUT, TMW, SH)                                                           \
+    MXK_PW3(LNAME, LAYOUT, TMW, 1, 0, false, false, SH, _s##SH)                                    \
+    MXK_PW3(LNAME, LAYOUT, TMW, 1, 0, true, false, SH, _s##SH##_xm)
+#define MXK_PW_CHS(TMW, SH)                                                                        \
+    MXK_PW_S(ch, CH, TMW, SH)                                                                      \
+    MXK_PW3(ch, CH, TMW, 1, 1, false, false, SH, _s##SH##_ln)                                      \
+    MXK_PW3(ch, CH, TMW, 1, 0, false, true, SH, _s##SH##_mul)                                      \
+    MXK_PW_CT(TMW, 1, SH, _s##SH)                                                                  \
+    MXK_PWB1(TMW, 1, false, SH, _s##SH) MXK_PWB1(TMW, 1, true, SH, _s##SH##_xm)
 #define MXK_PW(LNAME, LAYOUT, TMW)                                                                 \
     MXK_PW1(LNAME, LAYOUT, TMW, 1, false, false, ) MXK_PW1(LNAME, LAYOUT, TMW, 4, false, false, _k4) \
     MXK_PW1(LNAME, LAYOUT, TMW, 1, false, true, _xm) MXK_PW1(LNAME, LAYOUT, TMW, 4, false, true, _k4_xm)
 #define MXK_PW_LN(TMW) MXK_PW1(ch, CH, TMW, 1, 1, false, _ln) MXK_PW1(ch, CH, TMW, 4, 1, false, _k4_ln)
 // _k4_ln2: the LayerNorm statistics computed by the block itself (LN = 2)
 MXK_PW1(ch, CH, 2, 4, 2, false, _k4_ln2)
-#define MXK_PW_CT(TMW, KS, SUF)                                                                    \
-    extern "C" __global__ __launch_bounds__(256) void mx_pw_ch##TMW##SUF##_t(GemmArgs a) {          \
-        pw::body<pw::CH, TMW, KS, false, false, false, false, true>(a, blockIdx.x, gridDim.x, blockIdx.y);                             \
+#define MXK_PW_CT(TMW, KS, SH, SUF)                                                                \
+    extern "C" __global__ __launch_bounds__(256) void mx_pw_ch##TMW##SUF##_t(GemmArgs a) {         \
+        pw::body<pw::CH, TMW, KS, false, 0, false, false, true, false, -1, false, false, SH>(      \
+            a, blockIdx.x, gridDim.x, blockIdx.y);                                                 \
     }
 // mx_pw_ch<TMW>[_k4][_ln]_f_lo: with a LayerNorm of one wave-wide band of
 // the output rows (GemmArgs lo).
-#define MXK_PW_LO(TMW, KS, LN, SUF)                                                               \
+#define MXK_PW_LO(TMW, KS, LN, SH, SUF)                                                            \
     extern "C" __global__ __launch_bounds__(256) void mx_pw_ch##TMW##SUF##_f_lo(GemmArgs a) {      \
-        pw::body<pw::CH, TMW, KS, true, LN, false, false, false, true>(a, blockIdx.x, gridDim.x, blockIdx.y);                          \
+        pw::body<pw::CH, TMW, KS, true, LN, false, false, false, true, -1, false, false, SH>(      \
+            a, blockIdx.x, gridDim.x, blockIdx.y);                                                 \
     }
 #define MXK_PW_MUL(TMW) \
     MXK_PW2(ch, CH, TMW, 1, false, false, true, _mul) MXK_PW2(ch, CH, TMW, 4, false, false, true, _k4_mul)
+// mx_pw_chb<TMW>[_k4][_xm][_f]: channel-major over a folded batch (GemmArgs
+// fold; GateMm mode 0, whose channels are the batch)
+#define MXK_PWB1(TMW, KS, XM, SH, SUF)                                                             \
+    extern "C" __global__ __launch_bounds__(256) void mx_pw_chb##TMW##SUF(GemmArgs a) {            \
+        pw::body<pw::CH, TMW, KS, false, 0, XM, false, false, false, -1, true, false, SH>(         \
+            a, blockIdx.x, gridDim.x, 0);                                                          \
+    }                                                                                              \
+    extern "C" __global__ __launch_bounds__(256) void mx_pw_chb##TMW##SUF##_f(GemmArgs a) {        \
+        pw::body<pw::CH, TMW, KS, true, 0, XM, false, false, false, -1, true, false, SH>(          \
+            a, blockIdx.x, gridDim.x, 0);                                                          \
+    }
+#define MXK_PWB(TMW)                                                                               \
+    MXK_PWB1(TMW, 1, false, 1, ) MXK_PWB1(TMW, 4, false, 1, _k4)                                   \
+    MXK_PWB1(TMW, 1, true, 1, _xm) MXK_PWB1(TMW, 4, true, 1, _k4_xm)
 MXK_PW(ch, CH, 1)
 MXK_PW(ch, CH, 2)
 MXK_PW(ch, CH, 4)
-// mx_pw_chb<TMW>[_k4][_xm][_f]: channel-major over a folded batch (GemmArgs
-// fold; GateMm mode 0, whose channels are the batch)
-#define MXK_PWB1(TMW, KS, XM, SUF)                                                                  \
-    extern "C" __global__ __launch_bounds__(256) void mx_pw_chb##TMW##SUF(GemmArgs a) {             \
-        pw::body<pw::CH, TMW, KS, false, 0, XM, false, false, false, -1, true>(a, blockIdx.x, gridDim.x, 0); \
-    }                                                                                               \
-    extern "C" __global__ __launch_bounds__(256) void mx_pw_chb##TMW##SUF##_f(GemmArgs a) {         \
-        pw::body<pw::CH, TMW, KS, true, 0, XM, false, false, false, -1, true>(a, blockIdx.x, gridDim.x, 0); \
-    }
-#define MXK_PWB(TMW) \
-    MXK_PWB1(TMW, 1, false, ) MXK_PWB1(TMW, 4, false, _k4) MXK_PWB1(TMW, 1, true, _xm) MXK_PWB1(TMW, 4, true, _k4_xm)
 MXK_PWB(1)
 MXK_PWB(2)
 MXK_PWB(4)
@@ -727,42 +914,62 @@ MXK_PW_LN(4)
 MXK_PW_MUL(1)
 MXK_PW_MUL(2)
 MXK_PW_MUL(4)
-MXK_PW_CT(1, 1, )
-MXK_PW_CT(1, 4, _k4)
-MXK_PW_CT(2, 1, )
-MXK_PW_CT(2, 4, _k4)
-MXK_PW_CT(4, 1, )
-MXK_PW_CT(4, 4, _k4)
-MXK_PW_LO(1, 1, 0, )
-MXK_PW_LO(2, 1, 0, )
-MXK_PW_LO(2, 4, 0, _k4)
-MXK_PW_LO(2, 1, 1, _ln)
-MXK_PW_LO(2, 4, 1, _k4_ln)
-MXK_PW_LO(4, 1, 0, )
-MXK_PW_LO(4, 4, 0, _k4)
-MXK_PW_LO(4, 1, 1, _ln)
-MXK_PW_LO(4, 4, 1, _k4_ln)
+MXK_PW_CT(1, 1, 1, )
+MXK_PW_CT(1, 4, 1, _k4)
+MXK_PW_CT(2, 1, 1, )
+MXK_PW_CT(2, 4, 1, _k4)
+MXK_PW_CT(4, 1, 1, )
+MXK_PW_CT(4, 4, 1, _k4)
+MXK_PW_CHS(1, 2)
+MXK_PW_CHS(2, 2)
+MXK_PW_CHS(1, 4)
+MXK_PW_CHS(2, 4)
+MXK_PW_S(rw, RW, 1, 2)
+MXK_PW_S(rw, RW, 2, 2)
+MXK_PW_S(rw, RW, 1, 4)
+MXK_PW_S(rw, RW, 2, 4)
+MXK_PW_LO(1, 1, 0, 1, )
+MXK_PW_LO(2, 1, 0, 1, )
+MXK_PW_LO(2, 4, 0, 1, _k4)
+MXK_PW_LO(2, 1, 1, 1, _ln)
+MXK_PW_LO(2, 4, 1, 1, _k4_ln)
+MXK_PW_LO(4, 1, 0, 1, )
+MXK_PW_LO(4, 4, 0, 1, _k4)
+MXK_PW_LO(4, 1, 1, 1, _ln)
+MXK_PW_LO(4, 4, 1, 1, _k4_ln)
+MXK_PW_LO(1, 1, 0, 2, _s2)
+MXK_PW_LO(1, 1, 0, 4, _s4)
+MXK_PW_LO(2, 1, 0, 2, _s2)
+MXK_PW_LO(2, 1, 0, 4, _s4)
+MXK_PW_LO(2, 1, 1, 2, _s2_ln)
+MXK_PW_LO(2, 1, 1, 4, _s4_ln)
 
 // mx_pw_..._f[_lo]_e<EP>: a fused streaming kernel specialised for one
 // epilogue operand set (pw::EP_* mask), for the combinations the MAXIM
 // program launches most; the host takes one when it exists and the generic
 // _f kernel otherwise (the same arithmetic in the same order).
-#define MXK_PW_E(NAME, LAYOUT, TMW, KS, LN, XM, XMUL, LNO, EP)                                     \
-    extern "C" __global__ __launch_bounds__(256) void NAME##_e##EP(GemmArgs a) {                  \
-        pw::body<pw::LAYOUT, TMW, KS, true, LN, XM, XMUL, false, LNO, EP>(a, blockIdx.x, gridDim.x, blockIdx.y); \
+#define MXK_PW_ES(NAME, LAYOUT, TMW, KS, LN, XM, XMUL, LNO, FOLD, SH, EP)                          \
+    extern "C" __global__ __launch_bounds__(256) void NAME##_e##EP(GemmArgs a) {                   \
+        pw::body<pw::LAYOUT, TMW, KS, true, LN, XM, XMUL, false, LNO, EP, FOLD, false, SH>(        \
+            a, blockIdx.x, gridDim.x, FOLD ? 0 : blockIdx.y);                                      \
     }
+#define MXK_PW_E(NAME, LAYOUT, TMW, KS, LN, XM, XMUL, LNO, EP) \
+    MXK_PW_ES(NAME, LAYOUT, TMW, KS, LN, XM, XMUL, LNO, false, 1, EP)
 // NAME_e<EP>_x2: two independent launches of that kernel as one grid (the
 // first d.na blocks run d.a, the rest d.b; one batch each), so that two
 // steps too small to fill the chip share its CUs and one launch's tail. Both
 // parts run the same function, so they share its LDS.
-#define MXK_PW_X2(NAME, LAYOUT, TMW, KS, LN, XM, XMUL, LNO, EP)                                    \
-    extern "C" __global__ __launch_bounds__(256) void NAME##_e##EP##_x2(DualGemmArgs d) {         \
+#define MXK_PW_X2S(NAME, LAYOUT, TMW, KS, LN, XM, XMUL, LNO, SH, EP)                               \
+    extern "C" __global__ __launch_bounds__(256) void NAME##_e##EP##_x2(DualGemmArgs d) {          \
         if (blockIdx.x < d.na)                                                                     \
-            pw::body<pw::LAYOUT, TMW, KS, true, LN, XM, XMUL, false, LNO, EP>(d.a, blockIdx.x, d.na, 0); \
+            pw::body<pw::LAYOUT, TMW, KS, true, LN, XM, XMUL, false, LNO, EP, false, false, SH>(   \
+                d.a, blockIdx.x, d.na, 0);                                                         \
         else                                                                                       \
-            pw::body<pw::LAYOUT, TMW, KS, true, LN, XM, XMUL, false, LNO, EP>(d.b, blockIdx.x - d.na, \
-                                                                            gridDim.x - d.na, 0);  \
+            pw::body<pw::LAYOUT, TMW, KS, true, LN, XM, XMUL, false, LNO, EP, false, false, SH>(   \
+                d.b, blockIdx.x - d.na, gridDim.x - d.na, 0);                                      \
     }
+#define MXK_PW_X2(NAME, LAYOUT, TMW, KS, LN, XM, XMUL, LNO, EP) \
+    MXK_PW_X2S(NAME, LAYOUT, TMW, KS, LN, XM, XMUL, LNO, 1, EP)
 MXK_PW_E(mx_pw_ch2_ln_f_lo, CH, 2, 1, 1, false, false, true, 72)
 MXK_PW_E(mx_pw_ch4_k4_ln_f_lo, CH, 4, 4, 1, false, false, true, 72)
 MXK_PW_E(mx_pw_ch2_ln_f, CH, 2, 1, 1, false, false, false, 72)
@@ -789,9 +996,30 @@ MXK_PW_E(mx_pw_ch2_mul_f, CH, 2, 1, 0, false, true, false, 70)
 MXK_PW_E(mx_pw_ch2_k4_mul_f, CH, 2, 4, 0, false, true, false, 66)
 MXK_PW_E(mx_pw_ch2_k4_mul_f, CH, 2, 4, 0, false, true, false, 70)
 MXK_PW_E(mx_pw_rw2_k4_f, RW, 2, 4, 0, false, false, false, 65)
-extern "C" __global__ __launch_bounds__(256) void mx_pw_chb2_k4_f_e65(GemmArgs a) {
-    pw::body<pw::CH, 2, 4, true, 0, false, false, false, false, 65, true>(a, blockIdx.x, gridDim.x, 0);
-}
+MXK_PW_ES(mx_pw_chb2_k4_f, CH, 2, 4, 0, false, false, false, true, 1, 65)
+// with X shared by two or four waves
+#define MXK_PW_ESS(SH)                                                                  \
+    MXK_PW_ES(mx_pw_ch2_s##SH##_ln_f_lo, CH, 2, 1, 1, false, false, true, false, SH, 72) \
+    MXK_PW_ES(mx_pw_ch2_s##SH##_ln_f, CH, 2, 1, 1, false, false, false, false, SH, 72)   \
+    MXK_PW_ES(mx_pw_ch2_s##SH##_f_lo, CH, 2, 1, 0, false, false, true, false, SH, 64)    \
+    MXK_PW_ES(mx_pw_ch2_s##SH##_f_lo, CH, 2, 1, 0, false, false, true, false, SH, 66)    \
+    MXK_PW_ES(mx_pw_ch2_s##SH##_f, CH, 2, 1, 0, false, false, false, false, SH, 64)      \
+    MXK_PW_ES(mx_pw_ch2_s##SH##_f, CH, 2, 1, 0, false, false, false, false, SH, 66)      \
+    MXK_PW_ES(mx_pw_ch2_s##SH##_f, CH, 2, 1, 0, false, false, false, false, SH, 226)     \
+    MXK_PW_ES(mx_pw_ch2_s##SH##_mul_f, CH, 2, 1, 0, false, true, false, false, SH, 66)   \
+    MXK_PW_ES(mx_pw_ch2_s##SH##_mul_f, CH, 2, 1, 0, false, true, false, false, SH, 70)   \
+    MXK_PW_ES(mx_pw_rw2_s##SH##_f, RW, 2, 1, 0, false, false, false, false, SH, 65)      \
+    MXK_PW_ES(mx_pw_chb2_s##SH##_f, CH, 2, 1, 0, false, false, false, true, SH, 65)      \
+    MXK_PW_X2S(mx_pw_ch2_s##SH##_ln_f_lo, CH, 2, 1, 1, false, false, true, SH, 72)       \
+    MXK_PW_X2S(mx_pw_ch2_s##SH##_ln_f, CH, 2, 1, 1, false, false, false, SH, 72)         \
+    MXK_PW_X2S(mx_pw_ch2_s##SH##_f, CH, 2, 1, 0, false, false, false, SH, 226)
+MXK_PW_ESS(2)
+MXK_PW_ESS(4)
+MXK_PW_ES(mx_pw_ch1_s2_f_lo, CH, 1, 1, 0, false, false, true, false, 2, 66)
+MXK_PW_ES(mx_pw_ch1_s2_f, CH, 1, 1, 0, false, false, false, false, 2, 226)
+MXK_PW_ES(mx_pw_ch1_s2_mul_f, CH, 1, 1, 0, false, true, false, false, 2, 66)
+MXK_PW_ES(mx_pw_ch1_s2_mul_f, CH, 1, 1, 0, false, true, false, false, 2, 70)
+MXK_PW_X2S(mx_pw_ch1_s2_f, CH, 1, 1, 0, false, false, false, 2, 226)
 MXK_PW_E(mx_pw_rw4_k4_f, RW, 4, 4, 0, false, false, false, 65)
 MXK_PW_X2(mx_pw_ch2_ln_f_lo, CH, 2, 1, 1, false, false, true, 72)
 MXK_PW_X2(mx_pw_ch1_f, CH, 1, 1, 0, false, false, false, 226)
@@ -819,6 +1047,23 @@ extern "C" __global__ __launch_bounds__(256) void mx_pw_chb2_k4_f_e65__rw2_k4_f_
         pw::body<pw::RW, 2, 4, true, 0, false, false, false, false, 65, false, true>(d.b, blockIdx.x - d.na,
                                                                                       gridDim.x - d.na, 0, red);
 }
+// and with X shared by four waves
+extern "C" __global__ __launch_bounds__(256) void mx_pw_chb2_s4_xm__rw2_s4_xm_x2(DualGemmArgs d) {
+    __shared__ __align__(16) float pool[4 * 64 * 24];
+    if (blockIdx.x < d.na)
+        pw::body<pw::CH, 2, 1, false, 0, true, false, false, false, -1, true, true, 4>(d.a, blockIdx.x, d.na, 0, pool);
+    else
+        pw::body<pw::RW, 2, 1, false, 0, true, false, false, false, -1, false, true, 4>(d.b, blockIdx.x - d.na,
+                                                                                         gridDim.x - d.na, 0, pool);
+}
+extern "C" __global__ __launch_bounds__(256) void mx_pw_chb2_s4_f_e65__rw2_s4_f_e65_x2(DualGemmArgs d) {
+    __shared__ __align__(16) float pool[4 * 64 * 24];
+    if (blockIdx.x < d.na)
+        pw::body<pw::CH, 2, 1, true, 0, false, false, false, false, 65, true, true, 4>(d.a, blockIdx.x, d.na, 0, pool);
+    else
+        pw::body<pw::RW, 2, 1, true, 0, false, false, false, false, 65, false, true, 4>(d.b, blockIdx.x - d.na,
+                                                                                         gridDim.x - d.na, 0, pool);
+}
 // the out-projections of the two branches at the smallest resolutions: a
 // residual add (grid branch), and a residual add into a backward permutation
 // (block branch)
@@ -836,4 +1081,32 @@ extern "C" __global__ __launch_bounds__(256) void mx_pw_ch2_k4_x2(DualGemmArgs d
         pw::body<pw::CH, 2, 4, false, 0, false, false>(d.a, blockIdx.x, d.na, 0);
     else
         pw::body<pw::CH, 2, 4, false, 0, false, false>(d.b, blockIdx.x - d.na, gridDim.x - d.na, 0);
+}
+
+// The weights of a streaming GEMM in bf16 parts (SplitArgs): one block a
+// 16-row tile, one wave a chunk of 32 k's, once per executor.
+extern "C" __global__ __launch_bounds__(256) void mx_split_w(SplitArgs a) {
+    const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+    const int nC = (a.K + 31) / 32, row = blockIdx.x * 16 + i;
+    for (int c = threadIdx.x >> 6; c < nC; c += 4) {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int k = 32 * c + 16 * (e >> 2) + 4 * g + (e & 3);
+            v[e] = row < a.M && k < a.K ? a.w[(int64_t)row * a.K + k] : 0.0f;
+        }
+        u32x4 p[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint32_t h, m, l;
+            split2(v[2 * e], v[2 * e + 1], h, m, l);
+            p[0][e] = h;
+            p[1][e] = m;
+            p[2][e] = l;
+        }
+        u32x4 *o = (u32x4 *)a.out + ((int64_t)blockIdx.x * nC + c) * 192 + lane;
+        o[0] = p[0];
+        o[64] = p[1];
+        o[128] = p[2];
+    }
 }

@@ -1,0 +1,137 @@
+"""The streaming GEMMs' products from three-part bf16 operands (mx_pw_*), at
+the edges of every form: tiles whose waves share X in fours and twos (_s4, _s2),
+each wave its own, the split reduction (_k4) with whole and half chunks of 32
+k's, both layouts, ragged columns and rows.
+
+- Against a float64 product: each of the six products of 32 k's is added with
+  one rounding of the running sum, so after K / 32 chunks the sum has had at
+  most 6 K / 32 roundings of 2^-24 relative to sum |w x|, what the split drops
+  is below 3 * 2^-24 of it, and the split reduction and bias add 4 more: the
+  bound is (6 ceil(K / 32) + 7) 2^-24 (|W| |X| + |b|).
+- Operands the split cannot hold (infinities, NaN, the largest floats) and
+  sums that overflow give what fp32 arithmetic gives: the same infinities and
+  NaNs as the CPU path, and the finite outputs within the bound.
+"""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # op, shape, the form expected
+    ("conv", (64, 128, 208, 320), "ch2_s4"),   # two stages, four waves share
+    ("conv", (32, 64, 180, 364), "ch2_s2"),    # one stage, two waves share, a ragged column tile
+    ("conv", (96, 64, 180, 364), "ch2_s2"),    # three stages
+    ("conv", (64, 32, 180, 364), "ch2"),       # each wave its own X
+    ("conv", (48, 24, 180, 364), "ch2"),       # an odd superstep: half a chunk of zeros
+    ("conv", (16, 12, 33, 36), "ch1"),         # half a chunk, a partial weight tile
+    ("conv", (64, 40, 13, 20), "ch2_k4"),      # split: a quarter is half a chunk
+    ("conv", (192, 40, 13, 20), "ch2_k4"),     # split: quarters of three supersteps, half chunks at either end
+    ("conv", (512, 128, 9, 12), "ch2_k4"),     # split: four chunks a quarter
+    ("gate0", (32, 256, 280), "chb2_s4"),      # GateMm over tokens, a folded batch
+    ("gate0", (33, 64, 1000), "chb2_s2"),      # the same, an odd channel count
+    ("gate0", (32, 256, 96), "chb2_k4"),
+    ("gate1", (32, 258, 256), "rw2_s4"),       # GateMm over cells, ragged rows
+    ("gate1", (16, 2100, 64), "rw2_s2"),
+    ("gate1", (3, 37, 64), "rw2_k4"),
+]
+
+
+def _run(op, shape, poison=None):
+    from maxim_amd import hip as H
+    from maxim_amd import plan as P
+    rng = np.random.default_rng(sum(shape))
+    if op == "conv":
+        ci, co, h, w = shape
+        x = rng.standard_normal((ci, h, w)).astype(np.float32)
+        wt = rng.standard_normal((co, ci)).astype(np.float32)
+        b = rng.standard_normal(co).astype(np.float32)
+        o = P.make_op(P.CONV1X1, dst=1, src=0, w=0, bias=1, c_in=ci, c_out=co, h=h, wd=w)
+        bufs = [(ci, h, w), (co, h, w)]
+    else:
+        c, outer, inner = shape
+        mode = int(op[-1])
+        k = outer if mode == 0 else inner
+        x = rng.standard_normal((c, outer, inner)).astype(np.float32)
+        wt = rng.standard_normal((k, k)).astype(np.float32)
+        b = rng.standard_normal(k).astype(np.float32)
+        o = P.make_op(P.GATE_MM, dst=1, src=0, w=0, bias=1, c=c, mode=mode, p=[outer, inner])
+        bufs = [x.shape, x.shape]
+    if poison is not None:
+        poison(x, wt, rng)
+    cp = P.CustomPlan(bufs, [o], [wt, b], input=0, output=1)
+    gpu = H.Gpu(cp)
+    gpu.write_buf(0, x)
+    gpu.run_ops(0, 1)
+    got = gpu.read_buf(1).reshape(bufs[1])
+    kernel = gpu.launches()[0][1]
+    gpu.close()
+    return x, wt, b, got, kernel
+
+
+def _sums(op, x, wt, b):
+    """The op on float64 (or whatever x and wt are)."""
+    with np.errstate(all="ignore"):
+        if op == "conv":
+            return (wt @ x.reshape(x.shape[0], -1)).reshape(wt.shape[0], *x.shape[1:]) + b[:, None, None]
+        if op == "gate0":
+            return np.stack([wt @ c for c in x]) + b[:, None]
+        return x @ wt.T + b
+
+
+@pytest.mark.parametrize("op,shape,form", CASES)
+def test_split_products_against_64_bits(gpu_ok, op, shape, form):
+    x, wt, b, got, kernel = _run(op, shape)
+    print(op, shape, kernel, flush=True)
+    assert kernel.startswith("mx_pw_" + form), kernel
+    want = _sums(op, x.astype(np.float64), wt.astype(np.float64), b.astype(np.float64))
+    size = _sums(op, np.abs(x).astype(np.float64), np.abs(wt).astype(np.float64), np.abs(b).astype(np.float64))
+    k = wt.shape[1]
+    bound = (6 * -(-k // 32) + 7) * 2.0 ** -24 * size
+    worst = float((np.abs(got - want) / bound).max())
+    print("worst share of the bound %.3f" % worst)
+    assert worst <= 1.0
+
+
+@pytest.mark.parametrize("op,shape,form", CASES)
+def test_operands_the_split_cannot_hold(gpu_ok, op, shape, form):
+    big = np.float32(3.4e38)  # finite, but rounds to infinity in bf16
+
+    def poison(x, wt, rng):
+        # [streamed][k]; one poisoned operand per streamed element, so that no
+        # sum meets two infinities; one sign of weight, so an infinite input
+        # is an infinite sum
+        k = wt.shape[1]
+        v = x.reshape(k, -1).T if op == "conv" else x.transpose(0, 2, 1).reshape(-1, k) if op == "gate0" else x.reshape(-1, k)
+        v = v.copy()
+        wt[:] = np.abs(wt) + np.float32(0.5)
+        wt[-1, -1] = np.float32(3e38)
+        v[:, -1] = np.clip(v[:, -1], -0.5, 0.5)
+        bad = [np.inf, -np.inf, np.nan, big, -big, 2e38, 1e30, -1e30]
+        at = rng.choice(len(v), 2 * len(bad) + 2, replace=False)
+        for n, val in enumerate(bad + bad):
+            v[at[n], rng.integers(k - 1)] = np.float32(val)
+        v[at[-2], -1], v[at[-1], -1] = 10, -10  # overflows with the last weight
+        if op == "conv":
+            x[:] = v.T.reshape(x.shape)
+        elif op == "gate0":
+            x[:] = v.reshape(x.shape[0], x.shape[2], k).transpose(0, 2, 1)
+        else:
+            x[:] = v.reshape(x.shape)
+
+    x, wt, b, got, kernel = _run(op, shape, poison)
+    print(op, shape, kernel, flush=True)
+    want = _sums(op, x.astype(np.float64), wt.astype(np.float64), b.astype(np.float64))
+    size = _sums(op, np.abs(x).astype(np.float64), np.abs(wt).astype(np.float64), np.abs(b).astype(np.float64))
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    # where every partial sum is certainly in range the same value; a sum
+    # certainly past the range is infinite; between the two fp32 may do either
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf].astype(np.float32))
+    top = float(np.finfo(np.float32).max)
+    safe = np.isfinite(want) & (size < 0.5 * top)
+    bound = (6 * -(-wt.shape[1] // 32) + 7 + wt.shape[1]) * 2.0 ** -24 * size[safe]
+    assert np.isfinite(got[safe]).all() and (np.abs(got[safe] - want[safe]) <= bound).all()
+    over = np.isfinite(want) & (np.abs(want) > 1.01 * top) & (np.abs(want) >= 0.9 * size)
+    assert over.any() and np.isinf(got[over]).all()
