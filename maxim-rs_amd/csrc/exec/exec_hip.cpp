@@ -218,9 +218,9 @@ BlockMap mx_block_map(const mx_op &q, int32_t r1map) {
     return b;
 }
 
-// The LayerNorm tile kernel for c in {32, 64, 128}: c x P pixels per block,
+// The LayerNorm tile kernel for c in {32, 64, 128, 256}: c x P pixels per block,
 // the widest P (up to 8192 / c) that still gives four blocks per CU (two at
-// 128 channels, whose longer serial pass favours wider tiles), else the
+// 128 channels and more, whose longer serial pass favours wider tiles), else the
 // narrowest: the serial channel pass of a block is latency-bound, so small
 // planes want more blocks (measured at C4). Returns the pixels per block and
 // the name suffix.
@@ -1273,7 +1273,7 @@ void Gpu::build_launches(const mx_plan_desc *p, const std::vector<int64_t> &woff
                 int64_t per = MXK_BLOCK;  // pixels per block
                 const bool vec = o.hw % 4 == 0 && aligned(a.x, 16) && aligned(a.y, 16);
                 std::string kn = k;
-                if (vec && (o.c == 32 || o.c == 64 || o.c == 128)) {
+                if (vec && (o.c == 32 || o.c == 64 || o.c == 128 || o.c == 256)) {
                     const auto t = ln_tile(o.c, o.hw, cus);
                     kn = "mx_chan_ln_c" + std::to_string(o.c) + t.second;
                     per = t.first;
@@ -2896,7 +2896,7 @@ void Gpu::build_program(const mx_plan_desc *p) {
         ChanLnArgs sa = la;
         sa.y = stats;
         Launch sl;
-        if (ln.c == 64 || ln.c == 128) {
+        if (ln.c == 64 || ln.c == 128 || ln.c == 256) {
             // the LayerNorm kernels' LDS tile (measured faster than the
             // register loop from 64 channels up)
             const auto t = ln_tile(ln.c, ln.hw, cus);

@@ -360,9 +360,6 @@ __device__ void scale_add_stats_tile(const ScaleAddLnArgs &a) {
     }                                                                                               \
     extern "C" __global__ __launch_bounds__(MXK_BLOCK) void mx_chan_ln_stats_c##C##SUF(ChanLnArgs a) { \
         chan_ln_tile<C, P, true>(a, blockIdx.x);                                                    \
-    }                                                                                               \
-    extern "C" __global__ __launch_bounds__(MXK_BLOCK) void mx_chan_scale_add_stats_c##C##SUF(ScaleAddLnArgs a) { \
-        scale_add_stats_tile<C, P>(a);                                                              \
     }
 MXK_LN(32, 256, )
 MXK_LN(32, 128, _p128)
@@ -373,6 +370,28 @@ MXK_LN(64, 32, _p32)
 MXK_LN(128, 64, )
 MXK_LN(128, 32, _p32)
 MXK_LN(128, 16, _p16)
+// 256 channels (the wider models' lower levels and bottleneck): the register
+// loops below walk 256 dependent rows in 5 to 20 blocks, the tiles in 160 and
+// 640 (8 pixels each; bound by launch and latency). LayerNorm of 256 x 5120
+// 97.8 -> 11.4 us and of 256 x 1280 96.9 -> 6.9 us, their statistics 26.3 ->
+// 10.6 and 25.0 -> 6.1 us.
+MXK_LN(256, 32, )
+MXK_LN(256, 16, _p16)
+MXK_LN(256, 8, _p8)
+
+#define MXK_SCALE_ADD_LN(C, P, SUF)                                                                 \
+    extern "C" __global__ __launch_bounds__(MXK_BLOCK) void mx_chan_scale_add_stats_c##C##SUF(ScaleAddLnArgs a) { \
+        scale_add_stats_tile<C, P>(a);                                                              \
+    }
+MXK_SCALE_ADD_LN(32, 256, )
+MXK_SCALE_ADD_LN(32, 128, _p128)
+MXK_SCALE_ADD_LN(32, 64, _p64)
+MXK_SCALE_ADD_LN(64, 128, )
+MXK_SCALE_ADD_LN(64, 64, _p64)
+MXK_SCALE_ADD_LN(64, 32, _p32)
+MXK_SCALE_ADD_LN(128, 64, )
+MXK_SCALE_ADD_LN(128, 32, _p32)
+MXK_SCALE_ADD_LN(128, 16, _p16)
 
 // Any channel count, any alignment: reads x twice.
 extern "C" __global__ __launch_bounds__(MXK_BLOCK) void mx_chan_ln_any(ChanLnArgs a) {
