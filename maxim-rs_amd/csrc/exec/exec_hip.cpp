@@ -298,6 +298,7 @@ struct ConvCfg {
     int bm = 0, th = 0, ck = 0;
     int c3bm = 0, c3th = 0;  // the mx_c3 tile, when the op qualifies for it
     int wtc = 0;             // the Winograd kernel's tile columns (4 or 8), 0: not eligible
+    bool wany = false;       // ... in its any-width form
     int nsplit = 1;          // 4x4: slices of the split reduction (mx_conv4x4_*_s)
 };
 
@@ -314,6 +315,16 @@ int pick_wino(int64_t ci, int64_t co, int64_t h, int64_t w) {
     if (w % 32 == 0) return 16;
     if (w % 16 == 0) return 8;
     return w % 8 == 0 ? 4 : 0;
+}
+
+// Other widths on large planes: the any-width kernel (wino_u.h), where at most
+// half as many pixels again are computed as there are and the plane has at
+// least 2048 of them: 16 blocks of 128 pixels per 32 output channels, the
+// fewest that were tried. 128 -> 128 channels at 225x319 (28% more pixels
+// computed than there are) 231 -> 127 us.
+bool pick_wino_any(int64_t ci, int64_t co, int64_t h, int64_t w) {
+    if (ci < 16 || ci % 8 || co < 32 || w % 8 == 0 || 8 * h * w >= (1LL << 31)) return false;
+    return h * w >= 2048 && 2 * ((h + 3) / 4 * 4) * ((w + 31) / 32 * 32) <= 3 * h * w;
 }
 
 // F(2x2, 3x3)'s filter transform U = G g G^T (G = [1 0 0; 1/2 1/2 1/2;
@@ -342,6 +353,56 @@ std::vector<float> wino_weights(const float *w, int64_t co, int64_t ci) {
                 for (int nu = 0; nu < 4; ++nu) {
                     const int64_t lane = k * 16 + r, val = (nu * 2 + ks) * 2 + mi;
                     out[(size_t)((((mb * nch + ch) * 4 + xi) * 64 + lane) * 16 + val)] = (float)U[xi][nu];
+                }
+        }
+    return out;
+}
+
+// The nearest finite bf16 (ties to even) of a float, as a float; infinities
+// and NaNs stay what they are.
+float to_bf16(float x) {
+    uint32_t u;
+    memcpy(&u, &x, 4);
+    if ((u & 0x7f800000u) == 0x7f800000u)
+        u = u & 0x007fffffu ? u | 0x00400000u : u;
+    else if ((u & 0x7fff0000u) != 0x7f7f0000u)
+        u += 0x7fffu + ((u >> 16) & 1);
+    u &= 0xffff0000u;
+    memcpy(&x, &u, 4);
+    return x;
+}
+
+// The same for the any-width kernel (wino_u.h): U rounded once to float, then
+// as three bf16 parts (common.h), laid out per
+// (32-channel output block, 16-channel input chunk) as
+// [wave][nu][part][lane][8]: wave w holds the transform row xi = w, and lane
+// (k, r) = (lane / 32, lane % 32) its MFMA A operand, value e = U[4 w +
+// nu][channel 16 chunk + k + 2 e][output 32 block + r]. Two bf16 share a word
+// of the returned array.
+std::vector<float> wino_split_weights(const float *w, int64_t co, int64_t ci) {
+    static const double G[4][3] = {{1, 0, 0}, {0.5, 0.5, 0.5}, {0.5, -0.5, 0.5}, {0, 0, 1}};
+    const int64_t nmb = (co + 31) / 32, nch = (ci + 15) / 16;
+    std::vector<float> out((size_t)(nmb * nch * 4 * 4 * 3 * 64 * 4), 0.0f);
+    uint16_t *parts = reinterpret_cast<uint16_t *>(out.data());
+    for (int64_t m = 0; m < co; ++m)
+        for (int64_t c = 0; c < ci; ++c) {
+            const float *g = w + (m * ci + c) * 9;
+            double T[4][3];  // G g
+            for (int xi = 0; xi < 4; ++xi)
+                for (int t = 0; t < 3; ++t)
+                    T[xi][t] = G[xi][0] * (double)g[t] + G[xi][1] * (double)g[3 + t] + G[xi][2] * (double)g[6 + t];
+            const int64_t mb = m / 32, r = m % 32, ch = c / 16, e = (c % 16) / 2, k = c % 2;
+            for (int xi = 0; xi < 4; ++xi)
+                for (int nu = 0; nu < 4; ++nu) {
+                    float rest = (float)(T[xi][0] * G[nu][0] + T[xi][1] * G[nu][1] + T[xi][2] * G[nu][2]);
+                    for (int p = 0; p < 3; ++p) {
+                        const float h = to_bf16(rest);
+                        uint32_t bits;
+                        memcpy(&bits, &h, 4);
+                        const int64_t at = (((mb * nch + ch) * 4 + xi) * 4 + nu) * 3 + p;
+                        parts[(size_t)((at * 64 + k * 32 + r) * 8 + e)] = (uint16_t)(bits >> 16);
+                        rest = std::isfinite(h) ? rest - h : 0.0f;
+                    }
                 }
         }
     return out;
@@ -1025,7 +1086,13 @@ void Gpu::init(const mx_plan_desc *p) {
                 }
                 if (k3 && !std::getenv("MAXIM_NO_WINOGRAD")) {
                     ccfg[i].wtc = pick_wino(o.c_in, o.c_out, o.h, o.wd);
-                    if (ccfg[i].wtc) extra[i][2] = placev(wino_weights(w, o.c_out, o.c_in));
+                    if (ccfg[i].wtc) {
+                        extra[i][2] = placev(wino_weights(w, o.c_out, o.c_in));
+                    } else if (pick_wino_any(o.c_in, o.c_out, o.h, o.wd)) {
+                        ccfg[i].wtc = 16;
+                        ccfg[i].wany = true;
+                        extra[i][2] = placev(wino_split_weights(w, o.c_out, o.c_in));
+                    }
                 }
                 as_is(o.bias);
                 break;
@@ -1401,12 +1468,12 @@ void Gpu::build_launches(const mx_plan_desc *p, const std::vector<int64_t> &woff
                     q.kind = 2;
                     alt[i].push_back(l);
                     L.push_back(q);
-                } else if (k3 && cc.wtc && aligned(a.x, 16)) {
+                } else if (k3 && cc.wtc && (cc.wany || aligned(a.x, 16))) {
                     // Winograd F(2x2, 3x3): 32 output channels x TR x TC tiles
                     ConvArgs b = a;
                     b.w = X(i, 2);
                     b.cvec = aligned(a.y, 8) && a.ow % 2 == 0;
-                    Launch q = mk("mx_wino3_t" + std::to_string(cc.wtc));
+                    Launch q = mk("mx_wino3_t" + std::to_string(cc.wtc) + (cc.wany ? "_u" : ""));
                     const int trows = cc.wtc == 16 ? 4 : 8;  // output rows per block
                     q.g[0] = cdiv((int64_t)((a.oh + trows - 1) / trows) * ((a.ow + 2 * cc.wtc - 1) / (2 * cc.wtc)), 1);
                     q.g[1] = grid_yz((o.c_out + 31) / 32);

@@ -5,6 +5,7 @@
 #include "conv.h"
 #include "conv3.h"
 #include "wino.h"
+#include "wino_u.h"
 #include "pointwise.h"
 
 // The scratch of mxh_run_noalloc (channel-mean partial sums and LayerNorm

@@ -1,0 +1,90 @@
+"""The any-width Winograd 3x3 convolution (mx_wino3_t16_u) and its three-part
+bf16 products: chunks of 16 input channels with a half at the end, partial
+output blocks, rows and columns that end inside a block, at odd, even and
+4-aligned widths.
+
+Against float64: each of an output's nine groups of transformed sums carries the
+transforms' own roundings and at most 6 ceil(ci / 16) of its running sum, each
+2^-24; as 2-norms over random data that stays under 8e-8 sqrt(9 ci) of the
+result, four times what fp32 sums of 9 ci products give.
+Operands the parts cannot hold: the block forms its sums in fp32 instead, so the
+largest floats give finite, right outputs and an infinity spoils only the tiles
+that read it.
+"""
+
+import numpy as np
+import pytest
+
+from test_gpu_conv import unfused
+from test_gpu_pointwise import he, run_plan
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    (16, 32, 64, 51, "mx_wino3_t16_u"),
+    (40, 33, 90, 31, "mx_wino3_t16_u"),
+    (24, 40, 47, 61, "mx_wino3_t16_u"),
+    (32, 32, 46, 62, "mx_wino3_t16_u"),
+    (128, 64, 37, 60, "mx_wino3_t16_u"),
+]
+
+
+def conv64(x, wt, b):
+    co, ci = wt.shape[:2]
+    h, w = x.shape[1:]
+    p = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1)))
+    y = np.zeros((co, h * w))
+    for ky in range(3):
+        for kx in range(3):
+            y += wt[:, :, ky, kx].astype(np.float64) @ p[:, ky:ky + h, kx:kx + w].reshape(ci, -1)
+    return y.reshape(co, h, w) + b[:, None, None].astype(np.float64)
+
+
+def make(ci, co, h, w):
+    from maxim_amd import plan as P
+    rng = np.random.default_rng(ci + co + h + w)
+    x = rng.standard_normal((ci, h, w)).astype(np.float32)
+    wt = he(rng, (co, ci, 3, 3), 9 * ci)
+    b = (rng.standard_normal(co) * 0.1).astype(np.float32)
+    ops = [P.make_op(P.CONV3X3, dst=1, src=0, w=0, bias=1, c_in=ci, c_out=co, h=h, wd=w),
+           P.make_op(P.LRELU, dst=2, src=1, n=co * h * w, slope=0.2)]
+    bufs = [(ci, h, w), (co, h, w), (co, h, w)]
+    plain = P.CustomPlan(bufs[:2], ops[:1], [wt, b], input=0, output=1)
+    act = P.CustomPlan(bufs, ops, [wt, b], input=0, output=2)
+    return x, wt, b, plain, act
+
+
+@pytest.mark.parametrize("ci,co,h,w,kernel", CASES)
+def test_against_64_bits(gpu_ok, ci, co, h, w, kernel):
+    x, wt, b, plain, act = make(ci, co, h, w)
+    got, steps = run_plan(plain, {0: x}, 1)
+    want = conv64(x, wt, b)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print(steps, "relative error %.2e" % err, flush=True)
+    assert steps[0][2] == kernel
+    assert err <= 8e-8 * np.sqrt(9 * ci)
+    assert np.abs(got - want).max() <= 1e-4 * np.abs(want).max()
+    got, steps = run_plan(act, {0: x}, 2)
+    assert len(steps) == 1 and steps[0][2] == kernel + "_f_e16"
+    assert np.array_equal(got.view(np.uint32), unfused(act, {0: x}, 2).view(np.uint32))
+
+
+@pytest.mark.parametrize("ci,co,h,w,kernel", CASES)
+@pytest.mark.parametrize("bad", [np.float32(3.4e38), np.float32(-3.4e38), np.float32(np.inf), np.float32(np.nan)])
+def test_operands_the_parts_cannot_hold(gpu_ok, ci, co, h, w, kernel, bad):
+    x, wt, b, plain, _ = make(ci, co, h, w)
+    c, r, q = ci - 1, h - 2, w - 3
+    x[c, r, q] = bad
+    got, _ = run_plan(plain, {0: x}, 1)
+    clean = x.copy()
+    clean[c, r, q] = 0
+    want = conv64(clean, wt, b)
+    near = np.zeros((h, w), bool)
+    near[max(r - 3, 0):r + 4, max(q - 3, 0):q + 4] = True  # the 2x2 tiles whose 4x4 patches hold it
+    assert np.abs(got - want)[:, ~near].max() <= 1e-4 * np.abs(want).max()
+    if np.isfinite(bad):
+        want = conv64(x, wt, b)
+        top = 3.4e38 * np.abs(wt).max()
+        assert np.isfinite(got).all() and np.abs(got - want)[:, near].max() <= 1e-5 * top
+    else:
+        assert not np.isfinite(got[:, r - 1:r + 2, q - 1:q + 2]).any()
