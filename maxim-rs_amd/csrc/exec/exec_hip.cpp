@@ -1092,6 +1092,7 @@ void Gpu::init(const mx_plan_desc *p) {
                         ccfg[i].wtc = 16;
                         ccfg[i].wany = true;
                         extra[i][2] = placev(wino_split_weights(w, o.c_out, o.c_in));
+                        as_is(o.w);
                     }
                 }
                 as_is(o.bias);
@@ -1472,6 +1473,7 @@ void Gpu::build_launches(const mx_plan_desc *p, const std::vector<int64_t> &woff
                     // Winograd F(2x2, 3x3): 32 output channels x TR x TC tiles
                     ConvArgs b = a;
                     b.w = X(i, 2);
+                    if (cc.wany) b.wo = W(o.w);
                     b.cvec = aligned(a.y, 8) && a.ow % 2 == 0;
                     Launch q = mk("mx_wino3_t" + std::to_string(cc.wtc) + (cc.wany ? "_u" : ""));
                     const int trows = cc.wtc == 16 ? 4 : 8;  // output rows per block

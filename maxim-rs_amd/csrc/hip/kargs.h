@@ -274,6 +274,7 @@ struct ConvArgs {
     int32_t cvec;         // 1: y, u, r1, r2 are 16-byte aligned and ow % 4 == 0
     int32_t ksplit;       // split reduction (_s kernels): input-channel chunks per z-slice
     Epilogue e;
+    const float *wo;      // mx_wino3_t16_u: the filters as the plan has them, [co][ci][3][3]
 };
 
 // The sum of a split-reduction conv's partial outputs, in z order, plus the

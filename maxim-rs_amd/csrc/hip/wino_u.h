@@ -15,8 +15,10 @@
 // registers a position ahead). The output transform A^T . A runs in two halves:
 // the column half (over nu) in registers, the row half (over xi, across the
 // waves) after one exchange through LDS. A block with a non-finite sum (an
-// operand that bf16 parts cannot hold) forms its sums again in fp32, with U put
-// back together from its parts.
+// infinite or NaN operand, one that bf16 parts cannot hold, or transforms that
+// overflow) forms its outputs as direct sums of nine taps instead: the
+// transforms would turn an infinity into inf - inf = NaN, and reach pixels that
+// an output does not read.
 //
 // Bound by issue (the transforms and the split on the vector ALU, two waves a
 // SIMD at 230 VGPRs) and its last round of blocks. 128 -> 128 channels at
@@ -57,6 +59,7 @@ __device__ void body(const ConvArgs &a) {
     constexpr int HALO = CK * CS;
     constexpr int MS = 4 * 2 * BM * MP;
     constexpr int POOL = 2 * HALO > MS ? 2 * HALO : MS;
+    static_assert(BM * NT / 256 * 4 * 256 <= POOL, "the direct sums");
     static_assert(HP >= OW + 2 && HP % 2 == 0 && OW == 32, "eight rows of 32 words at a time");
     __shared__ __align__(16) float smem[POOL];
     __shared__ int bad[4];
@@ -136,12 +139,10 @@ __device__ void body(const ConvArgs &a) {
 
     f32x16 acc[4];
 
-    auto clear = [&]() {
 #pragma unroll
-        for (int nu = 0; nu < 4; ++nu)
+    for (int nu = 0; nu < 4; ++nu)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[nu][r] = 0.0f;
-    };
+        for (int r = 0; r < 16; ++r) acc[nu][r] = 0.0f;
     // this wave's row of B^T d of this lane's patches
     auto rows = [&](const float *Hs, float (&t)[8][4]) {
 #pragma unroll
@@ -164,7 +165,6 @@ __device__ void body(const ConvArgs &a) {
         return nu == 0 ? t[0] - t[2] : nu == 1 ? t[1] + t[2] : nu == 2 ? t[2] - t[1] : t[1] - t[3];
     };
 
-    clear();
     fetch_halo(0);
     fetch_u(0, 0);
     for (int chunk = 0; chunk < nchunk; ++chunk) {
@@ -207,45 +207,45 @@ __device__ void body(const ConvArgs &a) {
     const bool over = __builtin_amdgcn_ballot_w64(!__builtin_isfinite(fin)) != 0;
     if (lane == 0) bad[wave] = over;
     __syncthreads();
-    if (bad[0] | bad[1] | bad[2] | bad[3]) {
-        // the same sums by fp32 MFMAs (the block's four waves all come here)
-        clear();
-#pragma nounroll
-        for (int chunk = 0; chunk < nchunk; ++chunk) {
-            fetch_halo(chunk);
-            stage_halo(smem);
-            __syncthreads();
-            float t[8][4];
-            rows(smem, t);
-#pragma unroll
-            for (int nu = 0; nu < 4; ++nu) {
-                fetch_u(chunk, nu);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    float u = 0.0f;
-#pragma unroll
-                    for (int p = 2; p >= 0; --p) {
-                        const uint32_t d = ur[nu & 1][p][e / 2];
-                        u += __builtin_bit_cast(float, e % 2 ? d & 0xffff0000u : d << 16);
-                    }
-                    acc[nu] = __builtin_amdgcn_mfma_f32_32x32x2f32(u, col(t[e], nu), acc[nu], 0, 0, 0);
-                }
-            }
-            __syncthreads();
-        }
-    }
+    const bool direct = (bad[0] | bad[1] | bad[2] | bad[3]) != 0;
 
     // (.) A over nu in registers: u[dx] for this wave's transform row xi;
     // then the rows of all four waves meet in LDS as Ms[xi][dx][m][t].
-    __syncthreads();
+    if (!direct) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const float a0 = acc[0][r], a1 = acc[1][r], a2 = acc[2][r], a3 = acc[3][r];
-        const int m = r / 4 * 8 + 4 * lk + r % 4;
-        Ms[((wave * 2 + 0) * BM + m) * MP + lt] = a0 + a1 + a2;
-        Ms[((wave * 2 + 1) * BM + m) * MP + lt] = a1 - a2 - a3;
+        for (int r = 0; r < 16; ++r) {
+            const float a0 = acc[0][r], a1 = acc[1][r], a2 = acc[2][r], a3 = acc[3][r];
+            const int m = r / 4 * 8 + 4 * lk + r % 4;
+            Ms[((wave * 2 + 0) * BM + m) * MP + lt] = a0 + a1 + a2;
+            Ms[((wave * 2 + 1) * BM + m) * MP + lt] = a1 - a2 - a3;
+        }
+        __syncthreads();
+    } else {
+        // the 2x2 outputs of this thread's (output channel, tile) pairs, each
+        // its own sum in fp32 over the image and the untransformed filters,
+        // left in LDS for itself (tap by tap, channels innermost)
+#pragma nounroll
+        for (int q = 0; q < PAIRS; ++q) {
+            const int e = tid + q * 256, m = m0 + e / NT, t = e % NT;
+#pragma nounroll
+            for (int d = 0; d < 4; ++d) {
+                const int oy = oy0 + 2 * (t / TC) + d / 2, ox = ox0 + 2 * (t % TC) + d % 2;
+                float s = 0.0f;
+                if (m < a.co && oy < a.oh && ox < a.ow) {
+#pragma nounroll
+                    for (int tap = 0; tap < 9; ++tap) {
+                        const int iy = oy + tap / 3 - 1, ix = ox + tap % 3 - 1;
+                        if (iy < 0 || iy >= a.h || ix < 0 || ix >= a.wd) continue;
+                        const float *xi = a.x + (int64_t)iy * a.wd + ix;
+                        const float *wi = a.wo + (int64_t)m * a.ci * 9 + tap;
+#pragma nounroll
+                        for (int c = 0; c < a.ci; ++c) s = __builtin_fmaf(wi[c * 9], xi[(int64_t)c * plane], s);
+                    }
+                }
+                Ms[(q * 4 + d) * 256 + tid] = s;
+            }
+        }
     }
-    __syncthreads();
     // A^T . over xi, bias, epilogue, stores: thread -> (m, tile), tiles fastest
     // rows and columns may end inside the block
     const int64_t oplane = (int64_t)a.oh * a.ow;
@@ -254,16 +254,21 @@ __device__ void body(const ConvArgs &a) {
     for (int q = 0; q < PAIRS; ++q) {
         const int e = tid + q * 256, m = e / NT, t = e % NT;
         if (m0 + m >= a.co) continue;
-        float u[4][2];
-#pragma unroll
-        for (int xi = 0; xi < 4; ++xi)
-#pragma unroll
-            for (int dx = 0; dx < 2; ++dx) u[xi][dx] = Ms[((xi * 2 + dx) * BM + m) * MP + t];
         float y[2][2];
+        if (!direct) {
+            float u[4][2];
 #pragma unroll
-        for (int dx = 0; dx < 2; ++dx) {
-            y[0][dx] = u[0][dx] + u[1][dx] + u[2][dx];
-            y[1][dx] = u[1][dx] - u[2][dx] - u[3][dx];
+            for (int xi = 0; xi < 4; ++xi)
+#pragma unroll
+                for (int dx = 0; dx < 2; ++dx) u[xi][dx] = Ms[((xi * 2 + dx) * BM + m) * MP + t];
+#pragma unroll
+            for (int dx = 0; dx < 2; ++dx) {
+                y[0][dx] = u[0][dx] + u[1][dx] + u[2][dx];
+                y[1][dx] = u[1][dx] - u[2][dx] - u[3][dx];
+            }
+        } else {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) y[d / 2][d % 2] = Ms[(q * 4 + d) * 256 + tid];
         }
         const int oy = oy0 + 2 * (t / TC), ox = ox0 + 2 * (t % TC);
         if (ox >= a.ow) continue;

@@ -7,9 +7,9 @@ Against float64: each of an output's nine groups of transformed sums carries the
 transforms' own roundings and at most 6 ceil(ci / 16) of its running sum, each
 2^-24; as 2-norms over random data that stays under 8e-8 sqrt(9 ci) of the
 result, four times what fp32 sums of 9 ci products give.
-Operands the parts cannot hold: the block forms its sums in fp32 instead, so the
-largest floats give finite, right outputs and an infinity spoils only the tiles
-that read it.
+Operands the parts cannot hold: the block forms direct nine-tap sums instead, so
+the largest floats give finite, right outputs and an infinity is an infinity in
+the outputs that read it and nothing in the others.
 """
 
 import numpy as np
@@ -88,3 +88,40 @@ def test_operands_the_parts_cannot_hold(gpu_ok, ci, co, h, w, kernel, bad):
         assert np.isfinite(got).all() and np.abs(got - want)[:, near].max() <= 1e-5 * top
     else:
         assert not np.isfinite(got[:, r - 1:r + 2, q - 1:q + 2]).any()
+
+
+@pytest.mark.parametrize("ci,co,h,w,kernel", CASES)
+def test_infinities_and_the_largest_floats_as_direct_sums(gpu_ok, ci, co, h, w, kernel):
+    """What nine-tap sums give: an infinity is that infinity times a weight in
+    the outputs that read it and nothing in the others, opposite infinities and
+    NaNs are NaN, and neighbours of opposite sign past half the float range
+    (whose difference overflows) leave finite sums finite, within 9 ci roundings
+    of 2^-24 of the sum of magnitudes."""
+    x, wt, b, plain, _ = make(ci, co, h, w)
+    inf = np.float32(np.inf)
+    x[0, 3, 5], x[ci - 1, 3, 12], x[1, 3, 13] = inf, -inf, inf  # columns 11..14 read both of the last two
+    x[2, 20, 7] = np.nan
+    x[3, 30, 9], x[3, 30, 11], x[4, 30, 10] = 3e38, -3e38, 2.9e38
+    x[5, 0, 0], x[ci - 2, h - 1, w - 1] = -inf, inf
+    got, steps = run_plan(plain, {0: x}, 1)
+    assert steps[0][2] == kernel
+    with np.errstate(all="ignore"):
+        # (no zero weights, and padding is left out: no 0 * inf)
+        assert (wt != 0).all()
+        want = conv64(np.where(np.isfinite(x), x, 0), wt, b)
+        size = conv64(np.where(np.isfinite(x), np.abs(x), 0), np.abs(wt), np.abs(b))
+        kinds = [(conv64(m.astype(np.float32), np.where(s, wt > 0, wt < 0).astype(np.float32), 0 * b) +
+                  conv64(n.astype(np.float32), np.where(s, wt < 0, wt > 0).astype(np.float32), 0 * b)) > 0
+                 for m, n, s in ((x == inf, x == -inf, True), (x == inf, x == -inf, False))]
+        nan = conv64(np.isnan(x).astype(np.float32), np.ones_like(wt), 0 * b) > 0
+    nan |= kinds[0] & kinds[1]
+    want = np.where(nan, np.nan, np.where(kinds[0], np.inf, np.where(kinds[1], -np.inf, want)))
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~fin & ~nan], want[~fin & ~nan].astype(np.float32))
+    # the tiles beside the poisoned ones are Winograd sums, their own products'
+    # roundings through the transforms: 1e-4 of the largest ordinary output
+    near = size > 1e6
+    far, near = fin & ~near, fin & near
+    assert (np.abs(got[near] - want[near]) <= (9 * ci + 2) * 2.0 ** -24 * size[near]).all()
+    assert np.abs(got[far] - want[far]).max() <= 1e-4 * np.abs(want[far]).max()
