@@ -27,7 +27,7 @@ __device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
 // leave most of the vector ALU's issue slots free (the fp32 MFMA does not).
 // Parts below 2^-126 are flushed, so operands under 2^-110 lose their last
 // parts; an infinite, NaN or over-2^127.99 operand gives NaN in every product,
-// and a wave that finds a non-finite sum computes its tile again in fp32.
+// and a wave that finds a non-finite sum computes that sum again in fp32.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));

@@ -23,8 +23,9 @@
 // Two supersteps make the 32 k's of an MFMA, whatever their order, as the
 // weights are laid out in the same one. The six products of every 32 k's are
 // added smallest first, and the 32s in ascending order, in every form of the
-// kernel, so forms that differ in tile width or in how X reaches the matrix
-// cores agree to the bit.
+// kernel, and a sum that is not finite is formed in fp32 whatever its tile
+// holds, so forms that differ in tile width or in how X reaches the matrix
+// cores agree to the bit on any data.
 //
 // Measured on MI355X against the same kernels on fp32 MFMAs (which are bound by
 // the SIMDs' issue: MFMA and VALU add up there): GateMm over 256 tokens, 32
@@ -536,41 +537,46 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
         if (LNO) __syncthreads();
     }
     // An operand the split cannot hold (infinite, NaN, the largest floats)
-    // leaves NaN in its outputs, and sums may overflow: a wave with any
-    // non-finite sum forms its sums in fp32 instead, superstep by superstep.
-    float fin = 0.0f;
+    // leaves no finite sum in its outputs, and sums may overflow: a wave that
+    // has such sums forms them in fp32, superstep by superstep, and keeps the
+    // others, so that no output depends on what else is in its tile.
+    float top = 0.0f;  // (the maximum that keeps a NaN)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int mt = 0; mt < TMW; ++mt) {
-            fin = __builtin_fmaf(acc[j][mt][0], acc[j][mt][1], fin);
-            fin = __builtin_fmaf(acc[j][mt][2], acc[j][mt][3], fin);
-        }
-    if (__builtin_amdgcn_ballot_w64(!__builtin_isfinite(fin))) {
+        for (int mt = 0; mt < TMW; ++mt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) top = __builtin_elementwise_maximum(top, __builtin_fabsf(acc[j][mt][r]));
+    if (__builtin_amdgcn_ballot_w64(!__builtin_isfinite(top))) {
         const int first = SH > 1 ? -S0 : 0;
         const float *wp[TMW];
 #pragma unroll
         for (int mt = 0; mt < TMW; ++mt)
             wp[mt] = W + (int64_t)min(w0 + mt * 16 + i, wout - 1) * K + 4 * g + (S0 + first) * 16;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 4; ++j) {
+            f32x4 f[TMW];
 #pragma unroll
-            for (int mt = 0; mt < TMW; ++mt) acc[j][mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int mt = 0; mt < TMW; ++mt) f[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-        for (int s = 0; s < nSw; ++s) {
-            float4 wv[TMW];
-            load(first + s, xa, la, ma);
+            for (int s = 0; s < nSw; ++s) {
+                float4 wv[TMW];
+                load(first + s, xa, la, ma);
 #pragma unroll
-            for (int mt = 0; mt < TMW; ++mt) wv[mt] = ld4(wp[mt] + s * 16);
-            ready(xa, la, ma);
+                for (int mt = 0; mt < TMW; ++mt) wv[mt] = ld4(wp[mt] + s * 16);
+                ready(xa, la, ma);
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
+                for (int t = 0; t < 4; ++t)
 #pragma unroll
                     for (int mt = 0; mt < TMW; ++mt)
-                        acc[j][mt] = LAYOUT == CH ? mfma16(comp(xa[t], j), comp(wv[mt], t), acc[j][mt])
-                                                  : mfma16(comp(wv[mt], t), comp(xa[j], t), acc[j][mt]);
+                        f[mt] = LAYOUT == CH ? mfma16(comp(xa[t], j), comp(wv[mt], t), f[mt])
+                                             : mfma16(comp(wv[mt], t), comp(xa[j], t), f[mt]);
+            }
+#pragma unroll
+            for (int mt = 0; mt < TMW; ++mt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (!__builtin_isfinite(acc[j][mt][r])) acc[j][mt][r] = f[mt][r];
         }
     }
 

@@ -135,3 +135,44 @@ def test_operands_the_split_cannot_hold(gpu_ok, op, shape, form):
     assert np.isfinite(got[safe]).all() and (np.abs(got[safe] - want[safe]) <= bound).all()
     over = np.isfinite(want) & (np.abs(want) > 1.01 * top) & (np.abs(want) >= 0.9 * size)
     assert over.any() and np.isinf(got[over]).all()
+
+
+def _columns(op, x):
+    """x as [streamed element][k] (a copy)."""
+    k = x.shape[0] if op == "conv" else x.shape[1] if op == "gate0" else x.shape[2]
+    v = x.reshape(k, -1).T if op == "conv" else x.transpose(0, 2, 1).reshape(-1, k) if op == "gate0" else x.reshape(-1, k)
+    return v.copy()
+
+
+def _put(op, x, v):
+    """The inverse of _columns, into x."""
+    x[:] = v.T.reshape(x.shape) if op == "conv" else \
+        v.reshape(x.shape[0], x.shape[2], -1).transpose(0, 2, 1) if op == "gate0" else v.reshape(x.shape)
+
+
+def _rows(op, y):
+    """An output as [streamed element][weight row]."""
+    return y.reshape(y.shape[0], -1).T if op == "conv" else \
+        y.transpose(0, 2, 1).reshape(-1, y.shape[1]) if op == "gate0" else y.reshape(-1, y.shape[2])
+
+
+@pytest.mark.parametrize("op,shape,form", CASES)
+def test_sums_that_are_not_finite_leave_the_others(gpu_ok, op, shape, form):
+    """Infinite, NaN and overflowing operands change the outputs that they
+    reach and no bit of any other, whatever tile it shares with them."""
+    def poison(x, wt, rng):
+        v = _columns(op, x)
+        for n, val in enumerate((np.inf, np.nan, 3.4e38, -np.inf)):
+            v[3 + n * 11, n] = val
+        wt[2, 1] = np.float32(np.inf)
+        _put(op, x, v)
+
+    clean = _run(op, shape)[3]
+    got, kernel = _run(op, shape, poison)[3:]
+    print(op, shape, kernel, flush=True)
+    assert kernel.startswith("mx_pw_" + form), kernel
+    a, b = (_rows(op, y).copy() for y in (clean, got))
+    hit = np.zeros(a.shape, bool)
+    hit[[3, 14, 25, 36]], hit[:, 2] = True, True
+    assert not np.isfinite(b[:, 2]).any() and not np.isfinite(b[[3, 14, 36]]).any()
+    assert np.array_equal(a[~hit].view(np.uint32), b[~hit].view(np.uint32))
