@@ -373,7 +373,7 @@ float to_bf16(float x) {
 }
 
 // The same for the any-width kernel (wino_u.h): U rounded once to float, then
-// as three bf16 parts (common.h), laid out per
+// the three bf16 parts of 2^24 times it (common.h), laid out per
 // (32-channel output block, 16-channel input chunk) as
 // [wave][nu][part][lane][8]: wave w holds the transform row xi = w, and lane
 // (k, r) = (lane / 32, lane % 32) its MFMA A operand, value e = U[4 w +
@@ -394,7 +394,7 @@ std::vector<float> wino_split_weights(const float *w, int64_t co, int64_t ci) {
             const int64_t mb = m / 32, r = m % 32, ch = c / 16, e = (c % 16) / 2, k = c % 2;
             for (int xi = 0; xi < 4; ++xi)
                 for (int nu = 0; nu < 4; ++nu) {
-                    float rest = (float)(T[xi][0] * G[nu][0] + T[xi][1] * G[nu][1] + T[xi][2] * G[nu][2]);
+                    float rest = (float)(T[xi][0] * G[nu][0] + T[xi][1] * G[nu][1] + T[xi][2] * G[nu][2]) * 0x1p24f;
                     for (int p = 0; p < 3; ++p) {
                         const float h = to_bf16(rest);
                         uint32_t bits;

@@ -25,9 +25,14 @@ __device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
 // 256, the fp32 MFMA's 1.0e-7 / 1.4e-7 / 2.0e-7 / 2.9e-7. Six bf16 MFMAs take
 // 96 cycles of a SIMD for the 32 k's that eight fp32 ones take 256 for, and
 // leave most of the vector ALU's issue slots free (the fp32 MFMA does not).
-// Parts below 2^-126 are flushed, so operands under 2^-110 lose their last
-// parts; an infinite, NaN or over-2^127.99 operand gives NaN in every product,
-// and a wave that finds a non-finite sum computes that sum again in fp32.
+// Both operands are taken 2^24 times as large (kSplitScale): every bit of a
+// float, a subnormal one's too, is then in a part above 2^-126, below which
+// bf16 operands may be flushed, so no operand is too small to split exactly,
+// and sums 2^48 times as large are rounded like the plain ones wherever these
+// are normal floats. At the other end an infinite or NaN operand, one past
+// 2^104 or a sum past 2^80 leaves a sum that is not finite, which the wave
+// forms again in fp32.
+constexpr float kSplitScale = 0x1p24f, kUnsplit = 0x1p-48f;
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));

@@ -230,8 +230,8 @@ struct GemmArgs {
     const void *A3;       // the streaming kernels' weights, A split into bf16 parts (SplitArgs)
 };
 
-// A weight matrix [M][K] as the bf16 matrix cores' operands: each element's
-// three bf16 parts, [ceil(M / 16)][ceil(K / 32)][part][lane][8], lane l
+// A weight matrix [M][K] as the bf16 matrix cores' operands: the three bf16
+// parts of 2^24 times each element (common.h), [ceil(M / 16)][ceil(K / 32)][part][lane][8], lane l
 // holding row 16 t + l % 16 at k = 32 c + 4 (l / 16) + 0..3 and 16 more
 // (zeros past M and K).
 struct SplitArgs {

@@ -229,19 +229,23 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
             lv[1] = ld4(lbi + s * 16);
         }
     };
-    auto norm = [&](float4 *xv, const float4 *lv) {
+    auto norm = [&](float4 *xv, const float4 *lv, float sc) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const float w = comp(lv[0], q), c = comp(lv[1], q);
+            const float w = comp(lv[0], q) * sc, c = comp(lv[1], q) * sc;
             xv[q].x = (xv[q].x - lmean.x) * lrstd.x * w + c;
             xv[q].y = (xv[q].y - lmean.y) * lrstd.y * w + c;
             xv[q].z = (xv[q].z - lmean.z) * lrstd.z * w + c;
             xv[q].w = (xv[q].w - lmean.w) * lrstd.w * w + c;
         }
     };
-    // the loaded values to X's: normalised, or multiplied (mx_mul's a * b)
-    auto ready = [&](float4 *xv, const float4 *lv, const float4 *mv) {
-        if (LN) norm(xv, lv);
+    // the loaded values to X's: normalised, or multiplied (mx_mul's a * b),
+    // times the power of two sc
+    auto ready = [&](float4 *xv, const float4 *lv, const float4 *mv, float sc) {
+        if (LN) {
+            norm(xv, lv, sc);
+            return;
+        }
         if (XMUL) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -250,6 +254,13 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
                 xv[q].z = xv[q].z * mv[q].z;
                 xv[q].w = xv[q].w * mv[q].w;
             }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            xv[q].x = xv[q].x * sc;
+            xv[q].y = xv[q].y * sc;
+            xv[q].z = xv[q].z * sc;
+            xv[q].w = xv[q].w * sc;
         }
     };
     // the superstep's four k's of streamed element j of this lane, split
@@ -466,8 +477,8 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
         const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         auto step = [&](int cc, bool first) {
             const WParts w = wload(c0 + cc);
-            ready(xa, la, ma);
-            ready(xb, lb, mb);
+            ready(xa, la, ma, kSplitScale);
+            ready(xb, lb, mb, kSplitScale);
             if (first && par) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) xa[q] = zero4;
@@ -506,7 +517,7 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
         const int nst = nS / SH;
         auto stage = [&](int st, bool first) {
             WParts w = wload(st * SC);
-            ready(xa, la, ma);
+            ready(xa, la, ma, kSplitScale);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const Half p = split(xa, j);
@@ -547,7 +558,9 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
         for (int mt = 0; mt < TMW; ++mt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) top = __builtin_elementwise_maximum(top, __builtin_fabsf(acc[j][mt][r]));
+    float us = kUnsplit;  // what the sums are multiplied by
     if (__builtin_amdgcn_ballot_w64(!__builtin_isfinite(top))) {
+        us = 1.0f;
         const int first = SH > 1 ? -S0 : 0;
         const float *wp[TMW];
 #pragma unroll
@@ -564,7 +577,7 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
                 load(first + s, xa, la, ma);
 #pragma unroll
                 for (int mt = 0; mt < TMW; ++mt) wv[mt] = ld4(wp[mt] + s * 16);
-                ready(xa, la, ma);
+                ready(xa, la, ma, 1.0f);
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -576,12 +589,14 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
             for (int mt = 0; mt < TMW; ++mt)
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (!__builtin_isfinite(acc[j][mt][r])) acc[j][mt][r] = f[mt][r];
+                    acc[j][mt][r] = __builtin_isfinite(acc[j][mt][r]) ? acc[j][mt][r] * kUnsplit : f[mt][r];
         }
     }
 
     float *const red = pool;
+    __shared__ __align__(16) float rus[KS == 4 ? 4 : 1];  // each wave's us
     if (KS == 4) {
+        if (lane == 0) rus[wave] = us;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -595,6 +610,8 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
     const int lnspan = (KS == 1 ? a.lo.group : 1) * TW * a.lo.nband;  // rows with a LayerNorm
     const bool lnw = LNO && w0 >= a.lo.row0 && w0 < a.lo.row0 + lnspan;
     float4 vs[LNO && KS == 4 ? NK : 1];
+    float4 us4;
+    if (KS == 4) us4 = ld4(rus);
     if (FUSED && KS == 1) operands(0, 0);
 #pragma unroll
     for (int k = 0; k < NK; ++k) {
@@ -611,27 +628,17 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
         for (int u = 0; u < 4; ++u) {
             // CH: v[u] = Y[m][n + u] is acc[u][mt][x]; RW: v[u] = Y[row][c + u] is acc[x][mt][u]
             const int j = LAYOUT == CH ? u : x, r = LAYOUT == CH ? x : u;
+            // (a product with a power of two and one rounding of the sum)
+            const float bb = !has_bias ? 0.0f : LAYOUT == CH ? bias[mt].x : comp(bias[mt], u);
             if (KS == 1) {
-                v[u] = acc[j][mt][r];
+                v[u] = has_bias ? __builtin_fmaf(acc[j][mt][r], us, bb) : acc[j][mt][r] * us;
             } else {
                 const int q = (j * TMW + mt) * 4 + r;
-                float t = red[q * 64 + lane];
-                t = t + red[(NACC + q) * 64 + lane];
-                t = t + red[(2 * NACC + q) * 64 + lane];
-                v[u] = t + red[(3 * NACC + q) * 64 + lane];
-            }
-        }
-        if (has_bias) {
-            if (LAYOUT == CH) {
-                const float bb = bias[mt].x;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = bb + v[u];
-            } else {
-                const float4 bb = bias[mt];
-                v[0] = bb.x + v[0];
-                v[1] = bb.y + v[1];
-                v[2] = bb.z + v[2];
-                v[3] = bb.w + v[3];
+                float t = red[q * 64 + lane] * us4.x;
+                t = __builtin_fmaf(red[(NACC + q) * 64 + lane], us4.y, t);
+                t = __builtin_fmaf(red[(2 * NACC + q) * 64 + lane], us4.z, t);
+                t = __builtin_fmaf(red[(3 * NACC + q) * 64 + lane], us4.w, t);
+                v[u] = has_bias ? bb + t : t;
             }
         }
         if (FUSED) {
@@ -1105,7 +1112,7 @@ extern "C" __global__ __launch_bounds__(256) void mx_split_w(SplitArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             uint32_t h, m, l;
-            split2(v[2 * e], v[2 * e + 1], h, m, l);
+            split2(v[2 * e] * kSplitScale, v[2 * e + 1] * kSplitScale, h, m, l);
             p[0][e] = h;
             p[1][e] = m;
             p[2][e] = l;

@@ -1,6 +1,7 @@
 // 3x3 convolution (pad 1) at any image width by Winograd's minimal filtering
 // F(2x2, 3x3) (wino.h has the transforms and their matrices), its products
-// formed from three-part bf16 operands (common.h).
+// formed from three-part bf16 operands (common.h; the halo is scaled as it is
+// staged, U by the host).
 //
 // A block owns 32 output channels x 2 x 16 tiles (4 x 32 output pixels) and
 // walks the input channels in chunks of 16. Per chunk the input halo (6 x 34
@@ -118,10 +119,10 @@ __device__ void body(const ConvArgs &a) {
     };
     auto stage_halo = [&](float *Hs) {
 #pragma unroll
-        for (int i = 0; i < NW; ++i) Hs[wlds + 8 * (i / HH) * CS + i % HH * HP] = qw[i];
+        for (int i = 0; i < NW; ++i) Hs[wlds + 8 * (i / HH) * CS + i % HH * HP] = qw[i] * kSplitScale;
 #pragma unroll
         for (int i = 0; i < NET; ++i)
-            if (er0 + ER * i < HH) Hs[elds + ER * i * HP] = er[i];
+            if (er0 + ER * i < HH) Hs[elds + ER * i * HP] = er[i] * kSplitScale;
     };
     auto fetch_u = [&](int chunk, int nu) {
         const u32x4 *u = ublk + ((int64_t)(chunk * 4 + wave) * 4 + nu) * (3 * 64) + lane;
@@ -199,12 +200,13 @@ __device__ void body(const ConvArgs &a) {
                                                                   __builtin_bit_cast(bf16x8, vp[PV[k]]), acc[nu], 0, 0, 0);
         }
     }
-    float fin = 0.0f;
+    // (2^8 below the largest float, so that the output transform stays finite)
+    float top = 0.0f;
 #pragma unroll
     for (int nu = 0; nu < 4; ++nu)
 #pragma unroll
-        for (int r = 0; r < 16; r += 2) fin = __builtin_fmaf(acc[nu][r], acc[nu][r + 1], fin);
-    const bool over = __builtin_amdgcn_ballot_w64(!__builtin_isfinite(fin)) != 0;
+        for (int r = 0; r < 16; ++r) top = __builtin_elementwise_maximum(top, __builtin_fabsf(acc[nu][r]));
+    const bool over = __builtin_amdgcn_ballot_w64(!(top < 0x1p120f)) != 0;
     if (lane == 0) bad[wave] = over;
     __syncthreads();
     const bool direct = (bad[0] | bad[1] | bad[2] | bad[3]) != 0;
@@ -250,6 +252,7 @@ __device__ void body(const ConvArgs &a) {
     // rows and columns may end inside the block
     const int64_t oplane = (int64_t)a.oh * a.ow;
     const bool vec = a.cvec != 0;
+    const float us = direct ? 1.0f : kUnsplit;
 #pragma unroll
     for (int q = 0; q < PAIRS; ++q) {
         const int e = tid + q * 256, m = e / NT, t = e % NT;
@@ -278,7 +281,7 @@ __device__ void body(const ConvArgs &a) {
         for (int dy = 0; dy < 2; ++dy) {
             if (oy + dy >= a.oh) continue;
             const int64_t idx = ib + (int64_t)(oy + dy) * a.ow;
-            float v0 = bb + y[dy][0], v1 = bb + y[dy][1];
+            float v0 = __builtin_fmaf(y[dy][0], us, bb), v1 = __builtin_fmaf(y[dy][1], us, bb);
             if (EP == 16) {
                 v0 = v0 >= 0.0f ? v0 : a.e.slope * v0;
                 v1 = v1 >= 0.0f ? v1 : a.e.slope * v1;

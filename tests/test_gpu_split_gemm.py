@@ -10,7 +10,9 @@ k's, both layouts, ragged columns and rows.
   bound is (6 ceil(K / 32) + 7) 2^-24 (|W| |X| + |b|).
 - Operands the split cannot hold (infinities, NaN, the largest floats) and
   sums that overflow give what fp32 arithmetic gives: the same infinities and
-  NaNs as the CPU path, and the finite outputs within the bound.
+  NaNs as the CPU path, and the finite outputs within the bound; the outputs
+  that they do not reach keep every bit.
+- Small operands, subnormal ones too, keep all their bits.
 """
 
 import numpy as np
@@ -38,7 +40,7 @@ CASES = [
 ]
 
 
-def _run(op, shape, poison=None):
+def _run(op, shape, poison=None, bias=None):
     from maxim_amd import hip as H
     from maxim_amd import plan as P
     rng = np.random.default_rng(sum(shape))
@@ -60,6 +62,7 @@ def _run(op, shape, poison=None):
         bufs = [x.shape, x.shape]
     if poison is not None:
         poison(x, wt, rng)
+    b = b if bias is None else bias
     cp = P.CustomPlan(bufs, [o], [wt, b], input=0, output=1)
     gpu = H.Gpu(cp)
     gpu.write_buf(0, x)
@@ -176,3 +179,31 @@ def test_sums_that_are_not_finite_leave_the_others(gpu_ok, op, shape, form):
     hit[[3, 14, 25, 36]], hit[:, 2] = True, True
     assert not np.isfinite(b[:, 2]).any() and not np.isfinite(b[[3, 14, 36]]).any()
     assert np.array_equal(a[~hit].view(np.uint32), b[~hit].view(np.uint32))
+
+
+@pytest.mark.parametrize("which", ["x", "w"])
+@pytest.mark.parametrize("e", [-70, 100, 120])
+@pytest.mark.parametrize("op,shape,form", CASES)
+def test_operands_of_any_size(gpu_ok, op, shape, form, e, which):
+    """2^-e times the inputs (or weights) and the bias give 2^-e times the
+    outputs, down to subnormal operands: the same bits, but for the rounding of
+    sums (and of the four partial sums of a split reduction) that are
+    subnormal floats themselves, each within half of 2^-149."""
+    def grid(a, bits):  # whole numbers of 2^-bits, which stay floats at every e
+        return np.round(np.clip(a, -8, 8) * np.float32(2.0 ** bits)) * np.float32(2.0 ** -bits)
+
+    def scaled(s):
+        def poison(x, wt, rng):
+            x[:], wt[:] = grid(x, 20), grid(wt, 20)
+            (x if which == "x" else wt)[:] *= np.float32(s)
+        return poison
+
+    rng = np.random.default_rng(sum(shape))
+    b = grid(rng.standard_normal({"conv": shape[1], "gate0": shape[1], "gate1": shape[2]}[op]).astype(np.float32), 20)
+    base = _run(op, shape, scaled(1.0), b)[3]
+    got, kernel = _run(op, shape, scaled(2.0 ** -e), b * np.float32(2.0 ** -e))[3:]
+    print(op, shape, kernel, flush=True)
+    assert kernel.startswith("mx_pw_" + form), kernel
+    diff = np.abs(got.astype(np.float64) * 2.0 ** e - base).max()
+    print("largest difference %.1e" % diff)
+    assert np.abs(base).max() > 1 and diff <= 5 * 2.0 ** (e - 150)

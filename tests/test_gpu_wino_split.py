@@ -125,3 +125,25 @@ def test_infinities_and_the_largest_floats_as_direct_sums(gpu_ok, ci, co, h, w, 
     far, near = fin & ~near, fin & near
     assert (np.abs(got[near] - want[near]) <= (9 * ci + 2) * 2.0 ** -24 * size[near]).all()
     assert np.abs(got[far] - want[far]).max() <= 1e-4 * np.abs(want[far]).max()
+
+
+@pytest.mark.parametrize("which", ["x", "w"])
+@pytest.mark.parametrize("e", [-60, 100, 120])
+@pytest.mark.parametrize("ci,co,h,w,kernel", CASES)
+def test_operands_of_any_size(gpu_ok, ci, co, h, w, kernel, e, which):
+    """2^-e times the input (or the filters) and the bias give 2^-e times the
+    outputs, down to subnormal operands: the same bits, but for the rounding of
+    outputs that are subnormal floats themselves."""
+    from maxim_amd import plan as P
+    x, wt, b, plain, _ = make(ci, co, h, w)
+    # whole numbers of 2^-18, which stay floats at every e, as do their transforms
+    x, wt, b = (np.round(np.clip(a, -8, 8) * np.float32(2 ** 18)) * np.float32(2.0 ** -18) for a in (x, wt, b))
+    bufs, ops = [(ci, h, w), (co, h, w)], [P.Op.from_buffer_copy(plain.ops[0])]
+    s = np.float32(2.0 ** -e)
+    base, _ = run_plan(P.CustomPlan(bufs, ops, [wt, b], input=0, output=1), {0: x}, 1)
+    x, wt = (x * s, wt) if which == "x" else (x, wt * s)
+    got, steps = run_plan(P.CustomPlan(bufs, ops, [wt, b * s], input=0, output=1), {0: x}, 1)
+    assert steps[0][2] == kernel
+    diff = np.abs(got.astype(np.float64) * 2.0 ** e - base).max()
+    print("largest difference %.1e" % diff, flush=True)
+    assert np.abs(base).max() > 1 and diff <= 2.0 ** (e - 150)
