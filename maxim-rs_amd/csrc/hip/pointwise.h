@@ -66,7 +66,7 @@ __device__ __forceinline__ float comp(const float4 &v, int t) {
 // weight row past the edge only feeds output rows/columns of the MFMA tile
 // that are never stored, so no branch or select sits between the loads and
 // the matrix cores. The next stage's (or 32 k's) loads are in flight while one
-// multiplies.
+// (or its second half) multiplies.
 // The image index of blocked index e (0 <= e < plane) under map q (32-bit:
 // the host enables a map only below 2^31 elements).
 // n / d for n < 2^31, with the host's multiplier m and shift s for d.
@@ -218,11 +218,15 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
     for (int q = 0; q < 4; ++q) xq[q] = XMUL ? a.B2 + (int64_t)b * a.sB + (xp[q] - X) : nullptr;
     // superstep S0 + s of X, with what its normalisation or product needs
     auto load = [&](int s, float4 *xv, float4 *lv, float4 *mv) {
+        // SH = 1: an offset the compiler takes as it is; a pointer kept per load
+        // and advanced in the loop costs 10 to 20 VGPRs
+        int64_t at = s * xstep;
+        if (SH == 1) asm("" : "+s"(at));
 #pragma unroll
-        for (int q = 0; q < 4; ++q) xv[q] = ld4(xp[q] + s * xstep);
+        for (int q = 0; q < 4; ++q) xv[q] = ld4(xp[q] + at);
         if (XMUL) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) mv[q] = ld4(xq[q] + s * xstep);
+            for (int q = 0; q < 4; ++q) mv[q] = ld4(xq[q] + at);
         }
         if (LN) {
             lv[0] = ld4(lsc + s * 16);
@@ -295,24 +299,30 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
             for (int q = 0; q < 3; ++q) w.p[mt][q] = w3[mt][(c * 3 + q) * 64];
         return w;
     };
-    // the six products of streamed tile j's 32 k's with the weights, smallest
-    // first; first: the wave's first 32, which start from zero (an
-    // inline-constant accumulator instead of register moves)
-    auto mul = [&](int j, u32x4 xh, u32x4 xm, u32x4 xl, const WParts &w, bool first) {
+    // the six products of streamed tiles j .. j + n - 1's 32 k's with the
+    // weights, smallest first; first: the wave's first 32, which start from zero
+    // (an inline-constant accumulator instead of register moves)
+    struct Parts {
+        u32x4 h, m, l;
+    };
+    auto mul = [&](int j, int n, const Parts *x, const WParts &w, bool first) {
         const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-        auto one = [&](u32x4 x, int q, bool z) {
+        auto one = [&](u32x4 Parts::*part, int q, bool z) {
 #pragma unroll
-            for (int mt = 0; mt < TMW; ++mt) {
-                const f32x4 c = z ? zero : acc[j][mt];
-                acc[j][mt] = LAYOUT == CH ? mfma32(x, w.p[mt][q], c) : mfma32(w.p[mt][q], x, c);
-            }
+            for (int t = 0; t < n; ++t)
+#pragma unroll
+                for (int mt = 0; mt < TMW; ++mt) {
+                    const f32x4 c = z ? zero : acc[j + t][mt];
+                    acc[j + t][mt] =
+                        LAYOUT == CH ? mfma32(x[t].*part, w.p[mt][q], c) : mfma32(w.p[mt][q], x[t].*part, c);
+                }
         };
-        one(xh, 2, first);
-        one(xl, 0, false);
-        one(xm, 1, false);
-        one(xh, 1, false);
-        one(xm, 0, false);
-        one(xh, 0, false);
+        one(&Parts::h, 2, first);
+        one(&Parts::l, 0, false);
+        one(&Parts::m, 1, false);
+        one(&Parts::h, 1, false);
+        one(&Parts::m, 0, false);
+        one(&Parts::h, 0, false);
     };
     // The bias of this lane's outputs, fetched before the reduction.
     float4 bias[TMW];
@@ -473,7 +483,7 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
     float *const pool = XR ? xpool : pool_own;
     if constexpr (SH == 1) {
         // chunk cc of the wave's share: supersteps 2 cc - par and the next
-        const int nc = (nSw + par + 1) / 2, c0 = S0 >> 1;
+        const int nc = LN == 2 ? 1 : (nSw + par + 1) / 2, c0 = S0 >> 1;
         const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         auto step = [&](int cc, bool first) {
             const WParts w = wload(c0 + cc);
@@ -487,20 +497,30 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
 #pragma unroll
                 for (int q = 0; q < 4; ++q) xb[q] = zero4;
             }
-            u32x4 xs[4][3];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            auto parts = [&](int j) {
                 const Half p = split(xa, j), q = split(xb, j);
-                xs[j][0] = u32x4{p.h[0], p.h[1], q.h[0], q.h[1]};
-                xs[j][1] = u32x4{p.m[0], p.m[1], q.m[0], q.m[1]};
-                xs[j][2] = u32x4{p.l[0], p.l[1], q.l[0], q.l[1]};
-            }
-            if (cc + 1 < nc) {
+                return Parts{u32x4{p.h[0], p.h[1], q.h[0], q.h[1]}, u32x4{p.m[0], p.m[1], q.m[0], q.m[1]},
+                             u32x4{p.l[0], p.l[1], q.l[0], q.l[1]}};
+            };
+            // Two streamed tiles at a time: their accumulators' chains cover
+            // each other's latency, and the next two are split meanwhile. The
+            // next loads wait for the last two: with all four tiles split
+            // before and 32 more registers filling, the split reductions took
+            // 172 to 198 VGPRs, two waves a SIMD; now at most 168 and three
+            // (with the in-kernel statistics, one chunk, 121 and four; with a
+            // folded LayerNorm or Mul 168 to 220 and two). The 128-channel
+            // gMLP layer at 56x80, whose 560-block launches then fit at once:
+            // 76.9 -> 70.8 us.
+            const Parts xs[4] = {parts(0), parts(1), parts(2), parts(3)};
+            mul(0, 2, xs, w, first);
+            auto next = [&]() {
+                if (cc + 1 >= nc) return;
                 load(2 * cc + 2 - par, xa, la, ma);
                 load(min(2 * cc + 3 - par, nSw - 1), xb, lb, mb);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) mul(j, xs[j][0], xs[j][1], xs[j][2], w, first);
+            };
+            if (!XMUL) next();
+            mul(2, 2, xs + 2, w, first);
+            if (XMUL) next();  // (twice the registers)
         };
         step(0, true);
 #pragma unroll 1
@@ -534,8 +554,8 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const unsigned char *r = rd + cc * 12288 + j * 256;
-                    mul(j, *(const u32x4 *)r, *(const u32x4 *)(r + 4096), *(const u32x4 *)(r + 8192), cc ? wn : w,
-                        first && cc == 0);
+                    const Parts x = {*(const u32x4 *)r, *(const u32x4 *)(r + 4096), *(const u32x4 *)(r + 8192)};
+                    mul(j, 1, &x, cc ? wn : w, first && cc == 0);
                 }
             }
         };
@@ -559,7 +579,7 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
 #pragma unroll
             for (int r = 0; r < 4; ++r) top = __builtin_elementwise_maximum(top, __builtin_fabsf(acc[j][mt][r]));
     float us = kUnsplit;  // what the sums are multiplied by
-    if (__builtin_amdgcn_ballot_w64(!__builtin_isfinite(top))) {
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!__builtin_isfinite(top)) != 0, 0)) {
         us = 1.0f;
         const int first = SH > 1 ? -S0 : 0;
         const float *wp[TMW];
