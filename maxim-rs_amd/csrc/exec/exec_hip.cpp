@@ -794,7 +794,7 @@ private:
     // fold (channel-major, batch > 1): tile the batches' columns as one axis
     // (GemmArgs fold), so a batch of N columns that is not a multiple of 64
     // leaves no ragged tile per batch.
-    bool try_pw(int layout, const GemmArgs &a0, Launch &l, bool whole = false, bool fold = false) {
+    bool try_pw(int layout, const GemmArgs &a0, Launch &l, bool fold = false) {
         if (no_pw) return false;
         GemmArgs a = a0;
         fold = fold && layout == 0 && a.batch > 1 && a.N % 4 == 0 && a.N % 64 != 0 &&
@@ -810,9 +810,8 @@ private:
         const auto parts = w3.find({a.A, wout, (int64_t)a.K});
         if (parts == w3.end() || a.sA) return false;
         a.A3 = wdev + parts->second;
-        if (a.sA % 4 || a.sB % 4 || a.sC % 4 || a.batch > 65535) return false;
-        static const char *names[2][3] = {{"mx_pw_ch1", "mx_pw_ch2", "mx_pw_ch4"},
-                                          {"mx_pw_rw1", "mx_pw_rw2", "mx_pw_rw4"}};
+        if (a.sB % 4 || a.sC % 4 || a.batch > 65535) return false;
+        static const char *names[2][2] = {{"mx_pw_ch1", "mx_pw_ch2"}, {"mx_pw_rw1", "mx_pw_rw2"}};
         // Tile width, sharing and reduction split, from measurements on
         // MI355X: 32 weight outputs per wave in both layouts; four (two)
         // waves share X where the weight tiles come in fours (twos), so X is
@@ -827,12 +826,9 @@ private:
         const int64_t nib = (wout + 16 * tmw - 1) / (16 * tmw);
         const int64_t tiles = nib * ((slen + 63) / 64);
         if (tiles > 0x7fffffffLL) return false;
-        // whole: the reduction stays in one wave (a step whose epilogue
-        // normalises bands across several waves of a block, which needs them
-        // to hold whole tiles)
         const int64_t nbat = fold ? 1 : a.batch;
         const char *sh = shared_x(nib, a.K);
-        const bool k4 = !whole && a.K % 64 == 0 && ((a.K >= 128 && !*sh) || tiles * nbat < 4LL * cus);
+        const bool k4 = a.K % 64 == 0 && ((a.K >= 128 && !*sh) || tiles * nbat < 4LL * cus);
         l = mk(std::string(names[layout][ti]).insert(8, fold ? "b" : "") + (k4 ? "_k4" : sh));
         const int64_t grid = k4 ? tiles : (tiles + 3) / 4;
         if (grid > 0x7fffffffLL) return false;
@@ -851,7 +847,6 @@ private:
     // (weight matrix, rows, k's) -> its bf16 parts (GemmArgs A3), a byte offset in wdev
     std::map<std::tuple<const float *, int64_t, int64_t>, uint64_t> w3;
     std::vector<std::vector<Launch>> alt;
-    std::vector<char> whole_k;  // per op: keep a streaming GEMM's reduction in one wave
     bool no_pw = getenv("MAXIM_NO_PW") != nullptr;
     // keep the plan's order of arithmetic everywhere (fused = unfused to the bit)
     bool plan_order = getenv("MAXIM_PLAN_ORDER") != nullptr;
@@ -1172,25 +1167,6 @@ void Gpu::init(const mx_plan_desc *p) {
     if (repack && !std::getenv("MAXIM_NO_PAIR")) pg.plan_regions(p);
     pg.layout(p, repack);
     arena_len = pg.arena_len;
-    // A 1x1 conv whose step normalises (or takes the statistics of) output
-    // bands of 128 channels needs whole tiles per wave, so four waves of a
-    // block hold a band (64-channel bands fit one 64-wide wave with the
-    // split reduction). Up to 128 inputs, with at least two 32-wide tiles per
-    // SIMD, that costs the split reduction 1-2 us (measured at the MAXIM
-    // 112x160 shapes) and saves a LayerNorm or statistics pass; with fewer
-    // tiles (56x80) the whole reductions cost more than the pass. Its own
-    // launch takes the same form, so the fused and unfused passes still
-    // agree to the bit.
-    whole_k.assign(p->n_ops, 0);
-    for (const StepSpec &sp : pg.specs) {
-        const uint64_t g = sp.ln >= 0 ? sp.first + 1 : sp.first;
-        if (g >= p->n_ops || p->ops[g].kind != MX_OP_CONV1X1 || p->ops[g].c_in > 128) continue;
-        const mx_op &c = p->ops[g];
-        const int64_t band = sp.lno >= 0 ? p->ops[sp.lno].c : sp.so_nband > 0 ? sp.so_c : 0;
-        const int64_t tiles = (c.c_out + 31) / 32 * ((c.h * c.wd + 63) / 64);
-        if (band > 64 && tiles >= 8LL * cus) whole_k[g] = 1;
-    }
-
     // Size the pass before allocating it, and refuse with the numbers.
     // Scratch: channel-mean partial sums, then the statistics of a folded
     // LayerNorm ([2][hw], one step at a time).
@@ -1398,7 +1374,7 @@ void Gpu::build_launches(const mx_plan_desc *p, const std::vector<int64_t> &woff
                 set_args(l, a);
                 l.kind = 1;
                 Launch q;
-                if (try_pw(0, a, q, whole_k[i])) {
+                if (try_pw(0, a, q)) {
                     alt[i].push_back(l);
                     L.push_back(q);
                 } else {
@@ -1561,7 +1537,7 @@ void Gpu::build_launches(const mx_plan_desc *p, const std::vector<int64_t> &woff
                     set_args(l, a);
                     l.kind = 1;
                     Launch q;
-                    if (try_pw(0, a, q, false, true)) {
+                    if (try_pw(0, a, q, true)) {
                         alt[i].push_back(l);
                         L.push_back(q);
                     } else {
@@ -2611,14 +2587,12 @@ void Gpu::build_program(const mx_plan_desc *p) {
         // epilogue also normalises a 32-channel LayerNorm band then holds the
         // band in two waves of a block (44.8 -> 43.4 us for the 64 -> 32
         // out-projections at 448x640); not for steps that leave statistics.
-        if (e.r1 && sp.so_nband <= 0 && l.kind == 1 &&
-            (!strcmp(l.name, "mx_pw_ch2") || !strcmp(l.name, "mx_pw_ch2_mul"))) {
+        if (e.r1 && sp.so_nband <= 0 && l.kind == 1 && !strcmp(l.name, "mx_pw_ch2")) {
             GemmArgs a;
             memcpy(&a, l.a0, sizeof a);
             if (a.M <= 32 && a.batch == 1) {
                 const int64_t nib = (a.M + 15) / 16, tiles = nib * ((a.N + 63) / 64);
-                l.name = intern(std::string("mx_pw_ch1") + shared_x(nib, a.K) + (l.name + 9));
-                l.f = fn(l.name);
+                l.name = intern(std::string("mx_pw_ch1") + shared_x(nib, a.K));
                 l.g[0] = (unsigned)((tiles + 3) / 4);
             }
         }

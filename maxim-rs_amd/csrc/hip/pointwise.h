@@ -877,15 +877,17 @@ __device__ void body(const GemmArgs &a, int ux, int nx, int by, float *xpool = n
 // only), _f applies the fused epilogue. mx_pw_ch<TMW>[_k4]_t: the transposed
 // 2x2 stride-2 conv (rows ordered (ky, oc, kx), co and the input width in
 // GemmArgs co / wd, wd % 4 == 0).
+#define MXK_PWF(LNAME, LAYOUT, TMW, KS, LN, XM, XMUL, SH, SUF)                                     \
+    extern "C" __global__ __launch_bounds__(256) void mx_pw_##LNAME##TMW##SUF##_f(GemmArgs a) {    \
+        pw::body<pw::LAYOUT, TMW, KS, true, LN, XM, XMUL, false, false, -1, false, false, SH>(     \
+            a, blockIdx.x, gridDim.x, blockIdx.y);                                                 \
+    }
 #define MXK_PW3(LNAME, LAYOUT, TMW, KS, LN, XM, XMUL, SH, SUF)                                     \
     extern "C" __global__ __launch_bounds__(256) void mx_pw_##LNAME##TMW##SUF(GemmArgs a) {        \
         pw::body<pw::LAYOUT, TMW, KS, false, LN, XM, XMUL, false, false, -1, false, false, SH>(    \
             a, blockIdx.x, gridDim.x, blockIdx.y);                                                 \
     }                                                                                              \
-    extern "C" __global__ __launch_bounds__(256) void mx_pw_##LNAME##TMW##SUF##_f(GemmArgs a) {    \
-        pw::body<pw::LAYOUT, TMW, KS, true, LN, XM, XMUL, false, false, -1, false, false, SH>(     \
-            a, blockIdx.x, gridDim.x, blockIdx.y);                                                 \
-    }
+    MXK_PWF(LNAME, LAYOUT, TMW, KS, LN, XM, XMUL, SH, SUF)
 #define MXK_PW2(LNAME, LAYOUT, TMW, KS, LN, XM, XMUL, SUF) MXK_PW3(LNAME, LAYOUT, TMW, KS, LN, XM, XMUL, 1, SUF)
 #define MXK_PW1(LNAME, LAYOUT, TMW, KS, LN, XM, SUF) MXK_PW2(LNAME, LAYOUT, TMW, KS, LN, XM, false, SUF)
 // _s<SH>: X shared by SH waves of a block
@@ -953,13 +955,15 @@ MXK_PW_CT(2, 1, 1, )
 MXK_PW_CT(2, 4, 1, _k4)
 MXK_PW_CT(4, 1, 1, )
 MXK_PW_CT(4, 4, 1, _k4)
-MXK_PW_CHS(1, 2)
+// 16-wide tiles share X only where a step of 17 to 32 outputs with a residual
+// takes them (with_epilogue): the fused forms of two waves
+MXK_PWF(ch, CH, 1, 1, 0, false, false, 2, _s2)
+MXK_PWF(ch, CH, 1, 1, 0, true, false, 2, _s2_xm)
+MXK_PWF(ch, CH, 1, 1, 1, false, false, 2, _s2_ln)
+MXK_PWF(ch, CH, 1, 1, 0, false, true, 2, _s2_mul)
 MXK_PW_CHS(2, 2)
-MXK_PW_CHS(1, 4)
 MXK_PW_CHS(2, 4)
-MXK_PW_S(rw, RW, 1, 2)
 MXK_PW_S(rw, RW, 2, 2)
-MXK_PW_S(rw, RW, 1, 4)
 MXK_PW_S(rw, RW, 2, 4)
 MXK_PW_LO(1, 1, 0, 1, )
 MXK_PW_LO(2, 1, 0, 1, )
@@ -971,7 +975,6 @@ MXK_PW_LO(4, 4, 0, 1, _k4)
 MXK_PW_LO(4, 1, 1, 1, _ln)
 MXK_PW_LO(4, 4, 1, 1, _k4_ln)
 MXK_PW_LO(1, 1, 0, 2, _s2)
-MXK_PW_LO(1, 1, 0, 4, _s4)
 MXK_PW_LO(2, 1, 0, 2, _s2)
 MXK_PW_LO(2, 1, 0, 4, _s4)
 MXK_PW_LO(2, 1, 1, 2, _s2_ln)
