@@ -2727,14 +2727,15 @@ void Gpu::build_program(const mx_plan_desc *p) {
             return G;
         };
         const bool k4 = nm.find("_k4") != std::string::npos, lnn = nm.find("_ln") != std::string::npos;
-        int tmw = nm[8] - '0', G = fits(tmw, k4);
+        // (16-wide tiles with a folded LayerNorm have no such form)
+        int tmw = nm[8] - '0', G = tmw == 1 && lnn ? 0 : fits(tmw, k4);
         if (!G && (c == 32 || c == 64)) {
             tmw = (int)(c / 16);
             G = 1;
         }
         if (!G) return false;
         const int64_t nib = (a.M + 16 * tmw - 1) / (16 * tmw), tiles = nib * ((a.N + 63) / 64);
-        l.name = intern("mx_pw_ch" + std::to_string(tmw) + (k4 ? "_k4" : tmw > 2 || (tmw == 1 && lnn) ? "" : shared_x(nib, a.K)) +
+        l.name = intern("mx_pw_ch" + std::to_string(tmw) + (k4 ? "_k4" : tmw > 2 ? "" : shared_x(nib, a.K)) +
                         (lnn ? "_ln" : "") + "_f_lo");
         l.f = fn(l.name);
         l.g[0] = (unsigned)(k4 ? tiles : (tiles + 3) / 4);

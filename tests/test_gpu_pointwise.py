@@ -682,3 +682,46 @@ def test_layernorm_statistics_from_the_channel_scale(gpu_ok, c, h, w):
     err = float(np.abs(got.astype(np.float64) - want).max())
     print("max-abs vs CPU %.3g (max|cpu| %.3g)" % (err, float(np.abs(want).max())))
     assert err <= 1e-3, err
+
+
+@pytest.mark.parametrize("c,k,h,w", [
+    (32, 32, 64, 64),    # 16-wide tiles but for the LayerNorm of the output
+    (32, 96, 60, 36),    # the same, three chunks, a partial pixel tile
+    (16, 32, 32, 32),    # one 16-wide tile: the LayerNorm's own launch
+])
+@pytest.mark.parametrize("order", ["plan", "free"])
+def test_layernorms_before_and_after_a_narrow_dense(gpu_ok, monkeypatch, order, c, k, h, w):
+    """ChanLn -> Conv1x1 k->c (at most 32 outputs) -> Add -> ChanLn: the first
+    LayerNorm folded into the GEMM, the second in its epilogue where a tile
+    holds the band."""
+    from maxim_amd import plan as P
+    from maxim_amd import hip as H
+    set_order(monkeypatch, order)
+    rng = np.random.default_rng(c + k + h)
+    hw = h * w
+    X, L, R, T, Y, LN, Z = range(7)
+    bufs = [(k, h, w), (k, h, w)] + [(c, h, w)] * 5
+    ws = [he(rng, (c, k), k), (rng.standard_normal(c) * 0.1).astype(np.float32)]
+    for n in (k, c):
+        ws += [(1 + 0.1 * rng.standard_normal(n)).astype(np.float32), (0.1 * rng.standard_normal(n)).astype(np.float32)]
+    ops = [P.make_op(P.CHAN_LN, dst=L, src=X, scale=2, bias=3, c=k, hw=hw),
+           P.make_op(P.CONV1X1, dst=T, src=L, w=0, bias=1, c_in=k, c_out=c, h=h, wd=w),
+           P.make_op(P.ADD, dst=Y, src=T, src2=R, n=c * hw),
+           P.make_op(P.CHAN_LN, dst=LN, src=Y, scale=4, bias=5, c=c, hw=hw),
+           P.make_op(P.ADD, dst=Z, src=LN, src2=Y, n=c * hw)]
+    cp = P.CustomPlan(bufs, ops, ws, input=X, output=Z)
+    inputs = {X: rng.standard_normal(bufs[X]).astype(np.float32), R: rng.standard_normal(bufs[R]).astype(np.float32)}
+    got, steps = run_plan(cp, inputs, Z)
+    print("steps", steps)
+    assert any("_ln" in s[2] for s in steps) and (c == 16 or any(s[2].endswith("_ln_f_lo") for s in steps)), steps
+    gpu = H.Gpu(cp)
+    for bb, v in inputs.items():
+        gpu.write_buf(bb, v)
+    gpu.set_fusion(False)
+    gpu.run_ops(0, len(ops))
+    plain = gpu.read_buf(Z).reshape(bufs[Z])
+    gpu.close()
+    agree(got, plain, order, 1e-5 * (1 + float(np.abs(plain).max())), "passes")
+    err = float(np.abs(got.astype(np.float64) - oracle_plan(cp, inputs, Z)).max())
+    print("max-abs vs CPU %.3g" % err)
+    assert err <= 1e-3, err
