@@ -319,12 +319,23 @@ int pick_wino(int64_t ci, int64_t co, int64_t h, int64_t w) {
 
 // Other widths on large planes: the any-width kernel (wino_u.h), where at most
 // half as many pixels again are computed as there are and the plane has at
-// least 2048 of them: 16 blocks of 128 pixels per 32 output channels, the
-// fewest that were tried. 128 -> 128 channels at 225x319 (28% more pixels
-// computed than there are) 231 -> 127 us.
-bool pick_wino_any(int64_t ci, int64_t co, int64_t h, int64_t w) {
+// least 2048 of them (16 blocks of 128 pixels per 32 output channels), against
+// the implicit GEMM c (or mx_c3) that would run instead. Over 1372 shapes of 16
+// to 256 input and 32 to 384 output channels it is the faster, by up to 2.9
+// (128 -> 128 at 225x319 231 -> 127 us; 33 outputs computed as 64 at 300x203
+// still 1.04; mx_c3's shapes from 1.11), but for few input channels against the
+// GEMM's smallest tile, whose 64-pixel blocks fill the chip sooner. With 16, 24
+// or 40 of them (40 computed as 48), against a GEMM of no more waves of one
+// block per CU: 24 -> 96 at 37x60 7.5 us against 6.6, 40 -> 96 9.0 against
+// 8.8, 24 -> 320 at 52x100 (a third wave of 8 blocks) 15.2 against 13.9; where
+// the GEMM has a wave more, 24 -> 160 at 33x92 7.6 against 8.6.
+bool pick_wino_any(const ConvCfg &c, int64_t ci, int64_t co, int64_t h, int64_t w, int cus) {
     if (ci < 16 || ci % 8 || co < 32 || w % 8 == 0 || 8 * h * w >= (1LL << 31)) return false;
-    return h * w >= 2048 && 2 * ((h + 3) / 4 * 4) * ((w + 31) / 32 * 32) <= 3 * h * w;
+    if (h * w < 2048 || 2 * ((h + 3) / 4 * 4) * ((w + 31) / 32 * 32) > 3 * h * w) return false;
+    if (c.bm != 32 || c.th != 4 || ci == 32 || ci >= 48) return true;
+    const int64_t bands = (co + 31) / 32 * ((h + 3) / 4), per = cus > 0 ? cus : 256;
+    const int64_t wino = (bands * ((w + 31) / 32) + per - 1) / per, gemm = (bands * ((w + 15) / 16) + per - 1) / per;
+    return gemm > wino + (wino >= 3);
 }
 
 // F(2x2, 3x3)'s filter transform U = G g G^T (G = [1 0 0; 1/2 1/2 1/2;
@@ -1083,7 +1094,7 @@ void Gpu::init(const mx_plan_desc *p) {
                     ccfg[i].wtc = pick_wino(o.c_in, o.c_out, o.h, o.wd);
                     if (ccfg[i].wtc) {
                         extra[i][2] = placev(wino_weights(w, o.c_out, o.c_in));
-                    } else if (pick_wino_any(o.c_in, o.c_out, o.h, o.wd)) {
+                    } else if (pick_wino_any(cc, o.c_in, o.c_out, o.h, o.wd, cus)) {
                         ccfg[i].wtc = 16;
                         ccfg[i].wany = true;
                         extra[i][2] = placev(wino_split_weights(w, o.c_out, o.c_in));

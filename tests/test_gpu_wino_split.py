@@ -147,3 +147,22 @@ def test_operands_of_any_size(gpu_ok, ci, co, h, w, kernel, e, which):
     diff = np.abs(got.astype(np.float64) * 2.0 ** e - base).max()
     print("largest difference %.1e" % diff, flush=True)
     assert np.abs(base).max() > 1 and diff <= 2.0 ** (e - 150)
+
+
+@pytest.mark.parametrize("ci,co,h,w,kernel", [
+    # few input channels against the implicit GEMM's smallest tile: by the
+    # waves of one block per CU (256) of either
+    (24, 96, 37, 60, "mx_conv3x3_m32_t4"),    # 60 blocks against 120
+    (40, 96, 37, 60, "mx_conv3x3_m32_t4"),
+    (24, 320, 52, 100, "mx_conv3x3_m32_t4"),  # 520 (three waves) against 910 (four)
+    (24, 160, 33, 92, "mx_wino3_t16_u"),      # 135 against 270 (two)
+    (24, 64, 37, 60, "mx_wino3_t16_u"),       # another tile
+    (32, 96, 37, 60, "mx_wino3_t16_u"),       # as many input channels as are computed
+    (48, 96, 37, 60, "mx_wino3_t16_u"),
+])
+def test_the_choice_for_few_input_channels(gpu_ok, ci, co, h, w, kernel):
+    x, wt, b, plain, _ = make(ci, co, h, w)
+    got, steps = run_plan(plain, {0: x}, 1)
+    want = conv64(x, wt, b)
+    assert steps[0][2] == kernel
+    assert np.linalg.norm(got - want) <= 8e-8 * np.sqrt(9 * ci) * np.linalg.norm(want)
