@@ -792,6 +792,20 @@ private:
         fns_[name] = f;
         return f;
     }
+    // An optional kernel: null where the code object has none. The failed
+    // lookup's error is taken back: it would stay the thread's last error, which
+    // other users of the runtime read after their own calls.
+    hipFunction_t optional_fn(const std::string &name) {
+        auto it = fns_.find(name);
+        if (it != fns_.end()) return it->second;
+        hipFunction_t f = nullptr;
+        if (H.hipModuleGetFunction(&f, mod, name.c_str()) != 0) {
+            f = nullptr;
+            H.hipGetLastError();
+        }
+        fns_[name] = f;
+        return f;
+    }
     Launch mk(const std::string &kname) {
         Launch l;
         l.name = intern(kname);
@@ -3029,15 +3043,7 @@ void Gpu::pair_launches(const mx_plan_desc *p) {
         int space;  // 0 arena, 1 scratch
         uint64_t lo, hi;
     };
-    auto x2fn = [&](const char *name) -> hipFunction_t {
-        const std::string n = std::string(name) + "_x2";
-        auto it = fns_.find(n);
-        if (it != fns_.end()) return it->second;
-        hipFunction_t f = nullptr;
-        if (H.hipModuleGetFunction(&f, mod, n.c_str()) != 0) f = nullptr;
-        fns_[n] = f;
-        return f;
-    };
+    auto x2fn = [&](const char *name) { return optional_fn(std::string(name) + "_x2"); };
     // a kernel pairing two different launches: A__B_x2, A's blocks first
     auto hx2fn = [&](const char *a, const char *b) -> hipFunction_t {
         if (strncmp(b, "mx_pw_", 6)) return nullptr;
@@ -3372,15 +3378,9 @@ void Gpu::specialise(Launch &l) {
                    (a.e.act == MXK_ACT_LRELU ? 16 : 0) | (a.ymap.on ? 32 : 0) | (a.bias ? 64 : 0) |
                    (a.ymap.on && a.ymap.r1map ? 128 : 0);
     const std::string sn = nm + "_e" + std::to_string(ep);
-    auto it = fns_.find(sn);
-    hipFunction_t f = nullptr;
-    if (it != fns_.end()) {
-        f = it->second;
-    } else {
-        if (H.hipModuleGetFunction(&f, mod, sn.c_str()) != 0) f = nullptr;
-        fns_[sn] = f;
-        if (!f && std::getenv("MAXIM_EP_LOG")) fprintf(stderr, "maxim: no specialised %s\n", sn.c_str());
-    }
+    const bool known = fns_.count(sn) != 0;
+    const hipFunction_t f = optional_fn(sn);
+    if (!f && !known && std::getenv("MAXIM_EP_LOG")) fprintf(stderr, "maxim: no specialised %s\n", sn.c_str());
     if (!f) return;
     l.name = intern(sn);
     l.f = f;

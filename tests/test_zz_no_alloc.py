@@ -174,3 +174,16 @@ def test_noalloc_on_a_caller_stream_and_under_capture():
         dout.free()
         g.close()
         rt.hipStreamDestroy(s)
+
+
+def test_building_an_executor_leaves_no_runtime_error(gpu_ok):
+    """Kernels that the executor looks up and need not exist leave nothing in
+    the runtime's last error, where another user of the runtime (torch, at its
+    next launch) would find it."""
+    from maxim_amd import plan as P
+    from maxim_amd import hip as H
+    rt = _hip()
+    rt.hipGetLastError()
+    gpu = H.Gpu(P.Plan(weights("S-1"), 64, 64))
+    assert rt.hipGetLastError() == 0
+    gpu.close()
