@@ -1160,20 +1160,17 @@ void Gpu::init(const mx_plan_desc *p) {
     }
     blob.resize((blob.size() + 63) & ~(size_t)63);
     // The weights of the streaming GEMMs again, as the bf16 parts their kernels
-    // multiply: six bytes an element, split on the device from the blob.
-    struct Parts {
-        int64_t off, rows, k;
-        uint64_t at;
-    };
-    std::vector<Parts> parts;
-    wbytes = blob.size() * 4;
+    // multiply: six bytes an element, after the blob, split on the device by one
+    // launch over a table at the blob's end.
+    std::vector<SplitEntry> parts;
+    int64_t split_tiles = 0;
     {
         std::set<std::array<int64_t, 3>> seen;
         auto add = [&](int64_t off, int64_t rows, int64_t k) {
             if (off < 0 || rows <= 0 || k <= 0 || k % 16 || !seen.insert({off, rows, k}).second) return;
-            if (rows > 0x7fffffff || k > 0x7fffffff) return;
-            parts.push_back(Parts{off, rows, k, wbytes});
-            wbytes += (uint64_t)((rows + 15) / 16 * ((k + 31) / 32)) * 3072;
+            if (rows > 0x7fffffff || k > 0x7fffffff || split_tiles + rows / 16 >= 0x7fffffff) return;
+            parts.push_back(SplitEntry{off, 0, (int32_t)rows, (int32_t)k, (int32_t)split_tiles, 0});
+            split_tiles += (rows + 15) / 16;
         };
         for (uint64_t i = 0; i < p->n_ops; ++i) {
             const mx_op &o = p->ops[i];
@@ -1182,6 +1179,14 @@ void Gpu::init(const mx_plan_desc *p) {
             if (o.kind == MX_OP_GATE_MM) add(woff[o.w], o.p[o.mode == 0 ? 0 : 1], o.p[o.mode == 0 ? 0 : 1]);
         }
     }
+    const size_t table = blob.size();
+    blob.resize((table + parts.size() * sizeof(SplitEntry) / 4 + 63) & ~(size_t)63);
+    wbytes = blob.size() * 4;
+    for (SplitEntry &q : parts) {
+        q.out = wbytes;
+        wbytes += (uint64_t)((int64_t)((q.M + 15) / 16) * ((q.K + 31) / 32)) * 3072;
+    }
+    if (!parts.empty()) memcpy(&blob[table], parts.data(), parts.size() * sizeof(SplitEntry));
 
     // The fused program and the device layout it implies.
     n_ops = p->n_ops;
@@ -1238,13 +1243,13 @@ void Gpu::init(const mx_plan_desc *p) {
     check(H.hipMalloc(&ptr, scratch_len * 4), "hipMalloc(scratch)");
     scratch = static_cast<float *>(ptr);
     if (!blob.empty()) check(H.hipMemcpy(wdev, blob.data(), blob.size() * 4, kMemcpyH2D), "hipMemcpy(weights)");
-    for (const Parts &q : parts) {
-        const float *w = reinterpret_cast<const float *>(wdev) + q.off;
+    if (!parts.empty()) {
         Launch l = mk("mx_split_w");
-        set_args(l, SplitArgs{w, wdev + q.at, (int32_t)q.rows, (int32_t)q.k});
-        l.g[0] = cdiv(q.rows, 16);
+        set_args(l, SplitArgs{wdev, reinterpret_cast<const SplitEntry *>(wdev + table * 4), (int32_t)parts.size()});
+        l.g[0] = cdiv(split_tiles, 1);
         launch(l);
-        w3[{w, q.rows, q.k}] = q.at;
+        for (const SplitEntry &q : parts)
+            w3[{reinterpret_cast<const float *>(wdev) + q.w, (int64_t)q.M, (int64_t)q.K}] = q.out;
     }
     kernels = 0;
     sync();

@@ -227,17 +227,24 @@ struct GemmArgs {
     // The grid is then one-dimensional.
     int32_t fold, fsh;
     uint32_t fmul, pad2;
-    const void *A3;       // the streaming kernels' weights, A split into bf16 parts (SplitArgs)
+    const void *A3;       // the streaming kernels' weights, A split into bf16 parts (SplitEntry)
 };
 
 // A weight matrix [M][K] as the bf16 matrix cores' operands: the three bf16
 // parts of 2^24 times each element (common.h), [ceil(M / 16)][ceil(K / 32)][part][lane][8], lane l
 // holding row 16 t + l % 16 at k = 32 c + 4 (l / 16) + 0..3 and 16 more
 // (zeros past M and K).
-struct SplitArgs {
-    const float *w;
-    void *out;
+struct SplitEntry {
+    int64_t w;        // the matrix, in floats from the weights' base
+    uint64_t out;     // its parts, in bytes from there
     int32_t M, K;
+    int32_t first;    // its first block: one per 16 rows, in the table's order
+    int32_t pad;
+};
+struct SplitArgs {
+    void *base;
+    const SplitEntry *table;
+    int32_t n;
 };
 
 // Two independent streaming-GEMM launches of one kernel in one grid: blocks

@@ -1119,17 +1119,27 @@ extern "C" __global__ __launch_bounds__(256) void mx_pw_ch2_k4_x2(DualGemmArgs d
         pw::body<pw::CH, 2, 4, false, 0, false, false>(d.b, blockIdx.x - d.na, gridDim.x - d.na, 0);
 }
 
-// The weights of a streaming GEMM in bf16 parts (SplitArgs): one block a
-// 16-row tile, one wave a chunk of 32 k's, once per executor.
-extern "C" __global__ __launch_bounds__(256) void mx_split_w(SplitArgs a) {
+// The weights of every streaming GEMM in bf16 parts (SplitEntry): one block a
+// 16-row tile, one wave a chunk of 32 k's, one launch per executor (a launch
+// per matrix, 30 to 800 of them, took 3.4 us each).
+extern "C" __global__ __launch_bounds__(256) void mx_split_w(SplitArgs s) {
+    int lo = 0, hi = s.n;  // the last entry that starts at or before this block
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (s.table[mid].first <= (int)blockIdx.x) lo = mid;
+        else hi = mid;
+    }
+    const SplitEntry a = s.table[lo];
+    const float *w = (const float *)s.base + a.w;
     const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
-    const int nC = (a.K + 31) / 32, row = blockIdx.x * 16 + i;
+    const int tile = blockIdx.x - a.first;
+    const int nC = (a.K + 31) / 32, row = tile * 16 + i;
     for (int c = threadIdx.x >> 6; c < nC; c += 4) {
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int k = 32 * c + 16 * (e >> 2) + 4 * g + (e & 3);
-            v[e] = row < a.M && k < a.K ? a.w[(int64_t)row * a.K + k] : 0.0f;
+            v[e] = row < a.M && k < a.K ? w[(int64_t)row * a.K + k] : 0.0f;
         }
         u32x4 p[3];
 #pragma unroll
@@ -1140,7 +1150,7 @@ extern "C" __global__ __launch_bounds__(256) void mx_split_w(SplitArgs a) {
             p[1][e] = m;
             p[2][e] = l;
         }
-        u32x4 *o = (u32x4 *)a.out + ((int64_t)blockIdx.x * nC + c) * 192 + lane;
+        u32x4 *o = (u32x4 *)((unsigned char *)s.base + a.out) + ((int64_t)tile * nC + c) * 192 + lane;
         o[0] = p[0];
         o[64] = p[1];
         o[128] = p[2];
