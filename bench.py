@@ -13,16 +13,18 @@ in HBM when the timed region starts. Prints ONE JSON line:
                 `value`), one image at a time and as a serving loop
                 (mxh_run_batch, the host's staging overlapped with the
                 passes), `program_roofline` the fused program's own bound
-                (each launch's max(FLOPs / 157.3 TFLOP/s, bytes / 8 TB/s),
+                (each launch's max(FLOPs / its matrix peak, bytes / 8 TB/s),
                 summed) and the pass's fraction of it
-  roofline      the dominant kernel's achieved rate against its bound (fp32
-                MFMA 157.3 TFLOP/s or HBM 8 TB/s): algorithmic FLOPs or bytes
+  roofline      the dominant kernel's achieved rate against its bound (its
+                matrix peak or HBM 8 TB/s): algorithmic FLOPs or bytes
                 per launch over the average launch duration, from the HIP
                 start/stop events each dispatch records on the executor's
                 stream over K further (eager) passes; `traffic` = its measured
                 HBM-side bytes per launch (profiles/hbm_traffic_c4.md);
                 `frac_of_own_bound` the same launches against each one's own
-                roofline min(P, AI x B)
+                roofline min(P, AI x B). Matrix peaks: 157.3 TFLOP/s of fp32
+                MFMAs, 2500 / 6 for three-part bf16 products (mx_pw_*), 36 / 16
+                of these for Winograd, whose FLOPs count the direct form's
   cpu_baseline  the CPU path (oracle/, a C restatement of the reference's
                 src/exec_cpu.rs) timed on this host: the median of three full
                 C4 passes on every host core the process may use, plus one
@@ -194,20 +196,15 @@ def main():
             e[1] += 1
             e[2] += f
             e[3] += by
-            e[4] += launch_bound_ms(f, by, R)
+            e[4] += launch_bound_ms(f, by, R, R.matrix_peak(kn))
     ev_ms = float(np.median(ev_tot))
-    prog_bound_ms = sum(launch_bound_ms(f, by, R) for f, by in cost)
+    prog_bound_ms = sum(launch_bound_ms(f, by, R, R.matrix_peak(kn)) for (f, by), (_, kn) in zip(cost, launches))
 
     # The dominant kernel by device time; its arithmetic intensity picks the
     # roofline axis.
     kern, (tms, nl, fl, by, _) = max(per_kernel.items(), key=lambda kv: kv[1][0])
     avg_s = tms / nl / 1e3
-    ai = fl / by if by else 0.0
-    if ai >= R.RIDGE:
-        roof = {"bound": "mfma", "achieved": fl / nl / avg_s / 1e12, "peak": 157.3, "unit": "TFLOP/s"}
-    else:
-        roof = {"bound": "hbm", "achieved": by / nl / avg_s / 1e9, "peak": 8000.0, "unit": "GB/s"}
-    roof["frac"] = roof["achieved"] / roof["peak"]
+    roof = rate(fl, by, nl, avg_s, R, R.matrix_peak(kern))
     roof["traffic"] = traffic_per_launch(kern)
     roof["kernel"] = kern
     roof["avg_launch_us"] = avg_s * 1e6
@@ -278,8 +275,10 @@ def main():
         "e2e": e2e_rec,
         "program_roofline": {"bound_ms": prog_bound_ms, "kernel_ms": ev_ms, "launches": len(launches),
                              "frac": prog_bound_ms / ms_per_step,
-                             "what": "sum over the fused program's launches of max(FLOPs / 157.3 TFLOP/s, "
-                                     "bytes / 8 TB/s), algorithmic accounting; frac = bound / ms_per_step"},
+                             "what": "sum over the fused program's launches of max(FLOPs / matrix peak, "
+                                     "bytes / 8 TB/s), algorithmic accounting, the matrix peak 157.3 TFLOP/s of fp32 "
+                                     "MFMAs, 2500 / 6 of three-part bf16 products, 36 / 16 of these for Winograd; "
+                                     "frac = bound / ms_per_step"},
         "roofline": roof,
         "cpu_baseline": cpu,
         "device": device,
@@ -352,12 +351,12 @@ def c5_leg(w, R, name, steps=3):
             e[1] += 1
             e[2] += cost[k][0]
             e[3] += cost[k][1]
-            e[4] += launch_bound_ms(cost[k][0], cost[k][1], R)
+            e[4] += launch_bound_ms(cost[k][0], cost[k][1], R, R.matrix_peak(kn))
         kern, (tms, nl, fl, by, bd) = max(per.items(), key=lambda kv: kv[1][0])
         avg_s = tms / nl / 1e3
         fl_all = sum(c[0] for c in cost)
         by_all = sum(c[1] for c in cost)
-        dom = rate(fl, by, nl, avg_s, R)
+        dom = rate(fl, by, nl, avg_s, R, R.matrix_peak(kern))
         dom.update({"kernel": kern, "avg_launch_us": avg_s * 1e6, "launches_per_step": nl,
                     "share_of_pass": tms / tot, "frac_of_own_bound": bd / tms})
         # Per kernel: every memory-bound kernel (below the ridge) and the eight
@@ -366,12 +365,12 @@ def c5_leg(w, R, name, steps=3):
         for k, (t, n, f, b, _) in sorted(per.items(), key=lambda kv: -kv[1][0]):
             if n == 0 or t <= 0 or b <= 0:
                 continue
-            r = rate(f, b, n, t / n / 1e3, R)
+            r = rate(f, b, n, t / n / 1e3, R, R.matrix_peak(k))
             r.update({"kernel": k, "launches": n, "avg_us": 1e3 * t / n, "share": t / tot})
             rows.append(r)
         mem = [r for r in rows if r["bound"] == "hbm"]
         gemm = [r for r in rows if r["bound"] == "mfma"][:8]
-        bound_ms = sum(launch_bound_ms(c[0], c[1], R) for c in cost)
+        bound_ms = sum(launch_bound_ms(c[0], c[1], R, R.matrix_peak(kn)) for c, (_, kn) in zip(cost, launches))
         res = {"workload": "C5: %s, 4096x4096 RGB, one image per step" % name, "ms_per_image": ms,
                "images_per_s": 1e3 / ms, "steps": steps, "arena_gib": round(plan.arena_bytes / 2**30, 2),
                "kernel_ms_per_pass": tot, "tflops_effective": fl_all / (ms * 1e-3) / 1e12,
@@ -391,12 +390,13 @@ def c5_leg(w, R, name, steps=3):
         gpu.close()
 
 
-def rate(flops, nbytes, n, avg_s, R):
+def rate(flops, nbytes, n, avg_s, R, peak=None):
     """A kernel's achieved rate over n launches of avg_s seconds against the
-    peak its arithmetic intensity puts it under (fp32 MFMA above the ridge,
-    HBM below)."""
-    if nbytes and flops / nbytes >= R.RIDGE:
-        r = {"bound": "mfma", "achieved": flops / n / avg_s / 1e12, "peak": 157.3, "unit": "TFLOP/s"}
+    peak its arithmetic intensity puts it under (its matrix peak, by default
+    fp32 MFMA's, above the ridge, HBM below)."""
+    peak = peak or R.PEAK_FP32_MFMA
+    if nbytes and flops / nbytes >= peak / R.PEAK_HBM:
+        r = {"bound": "mfma", "achieved": flops / n / avg_s / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s"}
     else:
         r = {"bound": "hbm", "achieved": nbytes / n / avg_s / 1e9, "peak": 8000.0, "unit": "GB/s"}
     r["frac"] = r["achieved"] / r["peak"]
@@ -596,10 +596,10 @@ def gmlp_layer_range(plan):
     return first, last, x
 
 
-def launch_bound_ms(flops, nbytes, R):
-    """A launch's roofline time: the larger of its FLOPs at the fp32 MFMA peak
-    and its bytes at the HBM peak (ms)."""
-    return 1e3 * max(flops / R.PEAK_FP32_MFMA, nbytes / R.PEAK_HBM)
+def launch_bound_ms(flops, nbytes, R, peak=None):
+    """A launch's roofline time: the larger of its FLOPs at its matrix peak (by
+    default fp32 MFMA's) and its bytes at the HBM peak (ms)."""
+    return 1e3 * max(flops / (peak or R.PEAK_FP32_MFMA), nbytes / R.PEAK_HBM)
 
 
 if __name__ == "__main__":

@@ -3,14 +3,37 @@
 FLOPs = 2 x multiply-adds of the op as defined (no padding or halo work).
 Bytes = compulsory fp32 traffic: every input read once, the output written
 once, the weights read once. A fused kernel is charged its fused op's bytes.
-Peaks are MI355X's published dense figures.
+Peaks are MI355X's published dense figures, times what a kernel's form of the
+product makes of them (matrix_peak).
 """
 
 from . import plan as P
 
 PEAK_FP32_MFMA = 157.3e12   # FLOP/s
+PEAK_BF16_MFMA = 2.5e15
 PEAK_HBM = 8.0e12           # B/s
 RIDGE = PEAK_FP32_MFMA / PEAK_HBM
+
+# an fp32 product as six products of three-part bf16 operands
+PEAK_SPLIT = PEAK_BF16_MFMA / 6
+# F(2x2, 3x3): 16 products where the direct form has 36
+WINOGRAD = 36 / 16
+
+
+def matrix_peak(kernel):
+    """The rate of FLOPs (as the op defines them) at which the kernel's matrix
+    cores would be always busy."""
+    if kernel.startswith("mx_wino3_"):
+        return WINOGRAD * (PEAK_SPLIT if kernel.startswith("mx_wino3_t16_u") else PEAK_FP32_MFMA)
+    return PEAK_SPLIT if kernel.startswith("mx_pw_") else PEAK_FP32_MFMA
+
+
+def op_peak(op):
+    """The same for the kernels an op has at the model's shapes."""
+    if op.kind == P.CONV3X3:
+        return matrix_peak("mx_wino3_")
+    return matrix_peak("mx_pw_" if op.kind in (P.CONV1X1, P.CONVT2X2, P.GATE_MM) else "")
+
 
 GEMM_KINDS = {P.CONV1X1, P.CONV3X3, P.CONV4X4S2, P.CONVT2X2, P.GATE_MM}
 
@@ -63,7 +86,7 @@ def op_cost(op):
 def bound_s(op):
     """The op's roofline time: max(flops / peak, bytes / bandwidth)."""
     f, b = op_cost(op)
-    return max(f / PEAK_FP32_MFMA, b / PEAK_HBM)
+    return max(f / op_peak(op), b / PEAK_HBM)
 
 
 def plan_cost(plan):
