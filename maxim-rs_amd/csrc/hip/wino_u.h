@@ -61,7 +61,7 @@ __device__ void body(const ConvArgs &a) {
     constexpr int MS = 4 * 2 * BM * MP;
     constexpr int POOL = 2 * HALO > MS ? 2 * HALO : MS;
     static_assert(BM * NT / 256 * 4 * 256 <= POOL, "the direct sums");
-    static_assert(HP >= OW + 2 && HP % 2 == 0 && OW == 32, "eight rows of 32 words at a time");
+    static_assert(CK == 16 && HP >= OW + 2 && HP % 2 == 0 && OW == 32, "eight rows of 32 words at a time");
     __shared__ __align__(16) float smem[POOL];
     __shared__ int bad[4];
     float *Ms = smem;
@@ -87,42 +87,53 @@ __device__ void body(const ConvArgs &a) {
     // this block's transformed filters, [chunk][wave][nu][part][lane]
     const u32x4 *ublk = reinterpret_cast<const u32x4 *>(a.w) + ((int64_t)mb * nchunk) * (4 * 4 * 3 * 64);
 
-    // the halo loads of this thread: column wk of channels wc and wc + 8, and
-    // one edge column of channel ec in rows er0, er0 + ER, ...
+    // The halo loads of this thread: column wk of channels wc and wc + 8, and
+    // one edge column of channel ec in rows er0, er0 + ER, ... Addresses are
+    // clamped into the image, and what lies outside it is multiplied by 0
+    // instead of the operands' scale (an infinity read there is in the halo
+    // itself, so the block takes the direct sums). The last chunk may hold
+    // eight channels (c_in % 8 == 0): it reads them twice, the second time
+    // against U's zeros.
     const int wc = tid >> 5, wk = tid & 31;
     const int ec = tid / 2 % CK, side = tid & 1, er0 = tid / (CK * 2);
     const uint32_t plane = (uint32_t)a.h * (uint32_t)a.wd;  // 16 planes < 2^32, checked by the host
     const uint32_t wd = (uint32_t)a.wd;
-    const uint32_t woff = wc * plane + (uint32_t)(oy0 - 1) * wd + ox0 + wk;
-    const bool win = ox0 + wk < a.wd;
-    const uint32_t eoff = ec * plane + (uint32_t)(oy0 - 1 + er0) * wd + (side ? ox0 + OW : ox0 - 1);
-    const bool ein = side ? ox0 + OW < a.wd : ox0 > 0;
+    const uint32_t woff = wc * plane + min(ox0 + wk, a.wd - 1);
+    const int ecol = side ? ox0 + OW : ox0 - 1;
+    float wsc[HH], esc[NET];
+    uint32_t eoff[NET];
+#pragma unroll
+    for (int r = 0; r < HH; ++r)
+        wsc[r] = (unsigned)(oy0 - 1 + r) < (unsigned)a.h && ox0 + wk < a.wd ? kSplitScale : 0.0f;
+#pragma unroll
+    for (int i = 0; i < NET; ++i) {
+        const int iy = oy0 - 1 + er0 + ER * i;
+        esc[i] = (unsigned)iy < (unsigned)a.h && (unsigned)ecol < (unsigned)a.wd ? kSplitScale : 0.0f;
+        eoff[i] = (uint32_t)min(max(iy, 0), a.h - 1) * wd + min(max(ecol, 0), a.wd - 1);
+    }
     const int wlds = wc * CS + 1 + wk, elds = ec * CS + er0 * HP + (side ? OW + 1 : 0);
     float qw[NW], er[NET];
     u32x4 ur[2][3];  // two positions' filters, one in use and one on its way
     auto fetch_halo = [&](int chunk) {
-        const int cmax = a.ci - chunk * CK;
+        const bool half = a.ci - chunk * CK < CK;
         const float *xc = a.x + (int64_t)chunk * CK * plane;
+        const float *xw = xc + woff;
+        const int64_t q1 = half ? 0 : 8 * (int64_t)plane;
 #pragma unroll
         for (int i = 0; i < NW; ++i) {
-            const int iy = oy0 - 1 + i % HH;
-            qw[i] = 0.0f;
-            if (iy >= 0 && iy < a.h && win && wc + 8 * (i / HH) < cmax)
-                qw[i] = xc[woff + 8 * (i / HH) * plane + i % HH * wd];
+            const int iy = min(max(oy0 - 1 + i % HH, 0), a.h - 1);
+            qw[i] = xw[i / HH * q1 + (int64_t)iy * a.wd];
         }
+        const uint32_t ep = (half ? ec & 7 : ec) * plane;
 #pragma unroll
-        for (int i = 0; i < NET; ++i) {
-            const int r = er0 + ER * i, iy = oy0 - 1 + r;
-            er[i] = 0.0f;
-            if (r < HH && iy >= 0 && iy < a.h && ein && ec < cmax) er[i] = xc[eoff + ER * i * wd];
-        }
+        for (int i = 0; i < NET; ++i) er[i] = xc[ep + eoff[i]];
     };
     auto stage_halo = [&](float *Hs) {
 #pragma unroll
-        for (int i = 0; i < NW; ++i) Hs[wlds + 8 * (i / HH) * CS + i % HH * HP] = qw[i] * kSplitScale;
+        for (int i = 0; i < NW; ++i) Hs[wlds + 8 * (i / HH) * CS + i % HH * HP] = qw[i] * wsc[i % HH];
 #pragma unroll
         for (int i = 0; i < NET; ++i)
-            if (er0 + ER * i < HH) Hs[elds + ER * i * HP] = er[i] * kSplitScale;
+            if (er0 + ER * i < HH) Hs[elds + ER * i * HP] = er[i] * esc[i];
     };
     auto fetch_u = [&](int chunk, int nu) {
         const u32x4 *u = ublk + ((int64_t)(chunk * 4 + wave) * 4 + nu) * (3 * 64) + lane;
