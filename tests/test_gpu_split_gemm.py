@@ -213,3 +213,78 @@ def test_operands_of_any_size(gpu_ok, op, shape, form, e, which):
     diff = np.abs(got.astype(np.float64) * 2.0 ** e - base).max()
     print("largest difference %.1e" % diff)
     assert np.abs(base).max() > 1 and diff <= 5 * 2.0 ** (e - 150)
+
+
+@pytest.mark.parametrize("kind,ci,co,h,w,form", [
+    ("add", 64, 32, 256, 256, "ch1_s2_f"),      # 16-wide tiles, 32-wide when unfused
+    ("mul", 64, 32, 256, 256, "ch1_s2_mul_f"),
+    ("mul", 128, 128, 128, 160, "ch2_s4_mul_f"),
+    ("mul", 128, 64, 20, 28, "ch2_k4_mul_f"),
+    ("ln", 64, 128, 180, 364, "ch2_s4_ln_f"),
+    ("ln", 48, 24, 256, 260, "ch1_ln_f"),       # an odd superstep
+    ("ln", 128, 256, 20, 28, "ch2_k4_ln_f"),
+    ("t", 64, 32, 100, 200, "ch2_s4_t"),
+    ("t", 128, 16, 20, 28, "ch2_k4_t"),
+])
+def test_folded_operands_the_split_cannot_hold(gpu_ok, monkeypatch, kind, ci, co, h, w, form):
+    """Infinite, NaN and overflowing inputs where the streamed operand is formed
+    on the way in (a Mul, a LayerNorm) or the epilogue takes other tiles: the
+    unfused ops' bits. The transposed convolution: the CPU path's infinities and
+    NaNs, and its other values within the GEMM bar."""
+    from maxim_amd import hip as H
+    from maxim_amd import plan as P
+    from test_gpu_pointwise import fam, he, oracle_plan
+    monkeypatch.setenv("MAXIM_PLAN_ORDER", "1")  # fused = unfused to the bit
+    rng = np.random.default_rng(ci + co + h)
+    n = co * h * w
+    x = rng.standard_normal((ci, h, w)).astype(np.float32)
+    flat = x.reshape(ci, -1)
+    for k, val in enumerate((np.inf, -np.inf, np.nan, 3.4e38, -3e38, 1e35, 1e25)):
+        flat[rng.integers(ci), rng.choice(h * w, 2, replace=False)] = np.float32(val)
+    b = (rng.standard_normal(co) * 0.1).astype(np.float32)
+    X, F, M, T, R, Y = range(6)
+    bufs = [x.shape, x.shape, x.shape, (co, h, w), (co, h, w), (co, h, w)]
+    conv = dict(dst=T, src=X, w=0, bias=1, c_in=ci, c_out=co, h=h, wd=w)
+    add = P.make_op(P.ADD, dst=Y, src=T, src2=R, n=n)
+    ws = [he(rng, (co, ci), ci), b]
+    if kind == "t":
+        bufs, ws = [x.shape, (co, 2 * h, 2 * w)], [he(rng, (ci, co, 2, 2), ci), b]
+        ops, Y = [P.make_op(P.CONVT2X2, **dict(conv, dst=1))], 1
+    elif kind == "add":
+        ops = [P.make_op(P.CONV1X1, **conv), add]
+    elif kind == "mul":
+        ops = [P.make_op(P.MUL, dst=M, src=X, src2=F, n=x.size), P.make_op(P.CONV1X1, **dict(conv, src=M)), add]
+    else:
+        ws += [np.ones(ci, np.float32), np.zeros(ci, np.float32)]
+        ops = [P.make_op(P.CHAN_LN, dst=M, src=X, scale=2, bias=3, c=ci, hw=h * w),
+               P.make_op(P.CONV1X1, **dict(conv, src=M)), add]
+    cp = P.CustomPlan(bufs, ops, ws, input=X, output=Y)
+    inputs = {X: x}
+    if kind != "t":
+        inputs.update({F: rng.standard_normal(x.shape).astype(np.float32),
+                       R: rng.standard_normal((co, h, w)).astype(np.float32)})
+    outs = []
+    for fused in (True, False):
+        gpu = H.Gpu(cp)
+        gpu.set_fusion(fused)
+        for k, v in inputs.items():
+            gpu.write_buf(k, v)
+        gpu.run_ops(0, len(ops))
+        outs.append(gpu.read_buf(Y).reshape(cp.bufs[Y]))
+        if fused:
+            names = [fam(k) for _, k in gpu.launches()]
+        gpu.close()
+    got, plain = outs
+    print(kind, ci, co, h, w, names, "%d not finite" % (~np.isfinite(got)).sum(), flush=True)
+    assert "mx_pw_" + form in names
+    assert not np.isfinite(got).all() and np.isfinite(got).any()
+    assert np.array_equal(np.isnan(got), np.isnan(plain))
+    ok = ~np.isnan(got)
+    assert np.array_equal(got[ok].view(np.uint32), plain[ok].view(np.uint32))
+    if kind == "t":
+        with np.errstate(all="ignore"):
+            want = oracle_plan(cp, inputs, Y)
+        fin = np.isfinite(want)
+        assert np.array_equal(got[~fin & ok], want[~fin & ok]) and np.array_equal(np.isnan(got), np.isnan(want))
+        small = fin & (np.abs(want) < 1e3)
+        assert np.abs(got[small] - want[small]).max() <= 1e-4 * np.abs(want[small]).max()
