@@ -29,9 +29,9 @@
 //
 // Measured on MI355X against the same kernels on fp32 MFMAs (which are bound by
 // the SIMDs' issue: MFMA and VALU add up there): GateMm over 256 tokens, 32
-// channels at 448x640, 60.2 -> 34.4 us (mode 0) and 66.1 -> 34.1 us (mode 1),
-// 137 TFLOP/s; LayerNorm + Dense 128 -> 256 + GELU at 112x160 24.2 -> 14.7 us,
-// 32 -> 64 at 448x640 28.0 -> 23.0 us; a 640x448 S-3 pass 22.8 -> 19.5 ms.
+// channels at 448x640, 60.2 -> 35.3 us (mode 0) and 66.1 -> 34.5 us (mode 1),
+// 136 TFLOP/s; LayerNorm + Dense 128 -> 256 + GELU at 112x160 24.2 -> 14.7 us,
+// 32 -> 64 at 448x640 28.0 -> 23.0 us; a 640x448 S-3 pass 22.8 -> 19.1 ms.
 #pragma once
 
 #include "common.h"

@@ -22,9 +22,9 @@
 // an output does not read.
 //
 // Bound by issue (the transforms and the split on the vector ALU, two waves a
-// SIMD at 230 VGPRs) and its last round of blocks. 128 -> 128 channels at
-// 225x319: 231 us as implicit GEMM on fp32 MFMAs, 127 here (108 of kernel
-// time, 195 direct-equivalent TFLOP/s), error against 64 bits 6.1e-7 -> 2.9e-7.
+// SIMD at 224 VGPRs) and its last round of blocks. 128 -> 128 channels at
+// 225x319: 232 us as implicit GEMM on fp32 MFMAs, 126 here (110 of kernel
+// time, 192 direct-equivalent TFLOP/s), error against 64 bits 6.1e-7 -> 2.9e-7.
 // For the aligned widths the fp32 kernel of wino.h stays: with the same split
 // they measured 37.4 us against its 36.2 (32 channels, 448x640), 34.7 against
 // 34.8 (64, 224x320) and 41.3 against 37.4 (128, 112x160: 560 blocks over 512
