@@ -793,15 +793,17 @@ private:
         return f;
     }
     // An optional kernel: null where the code object has none. The failed
-    // lookup's error is taken back: it would stay the thread's last error, which
-    // other users of the runtime read after their own calls.
+    // lookup's error is taken back (unless an earlier one of the caller's waits to
+    // be read): it would stay the thread's last error, which other users of the
+    // runtime read after their own calls.
     hipFunction_t optional_fn(const std::string &name) {
         auto it = fns_.find(name);
         if (it != fns_.end()) return it->second;
         hipFunction_t f = nullptr;
+        const bool clean = H.hipPeekAtLastError() == 0;
         if (H.hipModuleGetFunction(&f, mod, name.c_str()) != 0) {
             f = nullptr;
-            H.hipGetLastError();
+            if (clean) H.hipGetLastError();
         }
         fns_[name] = f;
         return f;
